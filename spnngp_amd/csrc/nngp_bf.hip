@@ -52,6 +52,9 @@ constexpr int kCoopMaxWaves = 4;
 constexpr int kCoopMaxM = 64;
 constexpr int kCoopBlocks = 2048;  // logical blocks of the wavefront kernel
 constexpr int kGrpMaxM = 32;       // the row kernel's largest system
+// Waves of the row kernel: two a SIMD on 256 CUs, which is what its registers
+// allow, so that every block is resident and reads the matern table once.
+constexpr int kGrpWaves = 2048;
 constexpr int kRedThreads = 256;   // threads per block of the sum kernels
 constexpr int kRowsThreads = 1024; // threads per column of k_rows_sum
 constexpr int kRedBlocks = 1024;   // grid of the sum kernels (at most)
@@ -1124,35 +1127,86 @@ constexpr int kGrpSlots = 4 * kCoopMaxWaves;  // sites a block works on at once
 // neighbor coordinates, x then y.
 __host__ __device__ inline int grp_wave_doubles(int mm) { return 4 * 2 * mm; }
 
+// The pass's matern table (matern_piece): block o fills the pieces of octave
+// o from the series at their Chebyshev points; block 0 also writes the
+// Bessel-K loop divisors behind the table, for the entries outside it.
+// 36 blocks take about as long as one series evaluation; with every block of
+// the row kernel building a table for itself (and 16 coefficients an entry) a
+// pass took 261 us at n = 1e5, m = 15 and 1.99 ms at n = 5e5, m = 32; with
+// this launch before it, 140 us and 1.53 ms.
+constexpr int kMpThreads = 192;  // at least kMpSub * kMpN
+
+__global__ __launch_bounds__(kMpThreads) void k_matern_pieces(CovArgs c,
+                                                              double *out) {
+  __shared__ BesselTab bt;
+  __shared__ double fv[kMpSub * kMpN], cc[kMpSub * kMpN];
+  bessel_tab_fill(bt, c);
+  __syncthreads();
+  const int q = (int)threadIdx.x, o = (int)blockIdx.x;
+  const int pc = q / kMpN, j = q % kMpN;  // piece of the octave, node
+  if (q < kMpSub * kMpN) {
+    const double u = cospi((j + 0.5) / kMpN);
+    const double m = 1.0 + (pc + 0.5 + 0.5 * u) / kMpSub;
+    fv[q] = c.mnorm * xnu_bessel_k(ldexp(m, kMpOct0 + o), c, bt);
+  }
+  __syncthreads();
+  if (q < kMpSub * kMpN) {  // Chebyshev coefficient j of the piece
+    double s = 0.0;
+    for (int k = 0; k < kMpN; k++)
+      s = fma(fv[pc * kMpN + k], cospi(j * (k + 0.5) / kMpN), s);
+    cc[q] = s * (j == 0 ? 1.0 / kMpN : 2.0 / kMpN);
+  }
+  __syncthreads();
+  if (q < kMpSub * kMpN) {  // coefficient of (m - c)^j, u = 2 kMpSub (m - c)
+    double s = 0.0;
+    for (int k = j; k < kMpN; k++)
+      s = fma(cc[pc * kMpN + k], kChebMono.t[k][j], s);
+    out[(o * kMpSub + pc) * kMpN + j] = s * ldexp(1.0, 5 * j);
+  }
+  if (o == 0) {
+    const double *src = reinterpret_cast<const double *>(&bt);
+    for (int k = q; k < (int)(sizeof(BesselTab) / sizeof(double));
+         k += kMpThreads)
+      out[kMpLen + k] = src[k];
+  }
+}
+static_assert(2 * kMpSub == 32, "u = 2^5 (m - c)");
+
 // Covariance entries of the row kernel.  A lane evaluates about fifty per
 // site in fully unrolled code, so only the common path is inline: for the
-// matern (MAT) the pass's table, with near-coincident sites and x >= 64
-// (outside the table) out of line; otherwise the exponential, spherical and
-// gaussian.  The out-of-line series reads the parameters from the block's
-// LDS copy `al` (a reference to the kernel argument would make the kernel
-// keep a stack copy of it and read the inline path's fields from there).
+// matern (MAT) the pass's table, with coincident or nearly coincident sites
+// and x >= 64 (outside the table) out of line; otherwise the exponential,
+// spherical and gaussian.  The out-of-line series reads the parameters from
+// the block's LDS copy `al` (a reference to the kernel argument would make
+// the kernel keep a stack copy of it and read the inline path's fields from
+// there).
 __device__ __noinline__ double grp_matern_outside(double x, const CovArgs &al,
                                                   const BesselTab &bt) {
+  if (!(x > 0.0)) return al.s2;
   if (x > 700.0) return 0.0;
   return al.mnorm * xnu_bessel_k(x, al, bt);
 }
 
+// Where the row kernel's entries come from: the parameters and, for the
+// matern, their LDS copy, the table (LDS) and the divisors (device memory).
+struct GrpCov {
+  const CovArgs &a, &al;
+  const double *T;
+  const BesselTab &bt;
+};
+
 template <bool MAT>
-__device__ __forceinline__ double grp_corr(double d2, const CovArgs &a,
-                                           const CovArgs &al,
-                                           const BesselTab &bt,
-                                           const MaternTab &T) {
+__device__ __forceinline__ double grp_corr(double d2, const GrpCov &c) {
   if constexpr (MAT) {
-    const double x = nn_sqrt(d2) * a.phi;
-    if (!(x > 0.0)) return a.s2;
-    const int o = matern_tab_octave(x);
-    if ((unsigned)o >= (unsigned)kMatOct) return grp_matern_outside(x, al, bt);
-    return matern_tab_at(x, o, T);
+    const double x = nn_sqrt(d2) * c.a.phi;
+    const unsigned r = matern_piece(x);
+    if (r >= (unsigned)kMpRows) return grp_matern_outside(x, c.al, c.bt);
+    return matern_piece_at(x, r, c.T);
   } else {
-    switch (a.cov) {
-      case 0: return s2_corr<0>(d2, a);
-      case 1: return s2_corr<1>(d2, a);
-      default: return s2_corr<3>(d2, a);
+    switch (c.a.cov) {
+      case 0: return s2_corr<0>(d2, c.a);
+      case 1: return s2_corr<1>(d2, c.a);
+      default: return s2_corr<3>(d2, c.a);
     }
   }
 }
@@ -1206,9 +1260,7 @@ __device__ __forceinline__ void grp_in_xy(const BfProblem &P, int u, int i,
 // e; false when a pivot or F is not positive.
 template <int MM, bool MAT>
 __device__ inline bool grp_site(const BfArgs &A, const BfProblem &P,
-                                const CovArgs &c, const CovArgs &al,
-                                const BesselTab &bt,
-                                const MaternTab &mt, double *px, double *py,
+                                const GrpCov &gc, double *px, double *py,
                                 int i, bool valid, const GrpIn &in, int i2,
                                 bool valid2, GrpIn &in2, int u, double &F,
                                 double (&e)[kMaxNZ]) {
@@ -1217,6 +1269,7 @@ __device__ inline bool grp_site(const BfArgs &A, const BfProblem &P,
   // otherwise be hoisted out of the caller's site loop as lane masks, more
   // than the SGPR file holds
   u = lane_opaque(u);
+  const CovArgs &c = gc.a;
   const int cnt = in.cnt, off = in.off, ida = in.ida, idb = in.idb;
   const double2 qa = in.qa, qb = in.qb, s = in.s;
   const bool ina = u < cnt, inb = R == 2 && u + 16 < cnt;
@@ -1234,20 +1287,20 @@ __device__ inline bool grp_site(const BfArgs &A, const BfProblem &P,
     constexpr int l = decltype(lc)::value;
     S.ra[l] = l == u ? (ina ? c.diag : 1.0) : 0.0;
     if (l < u && ina)
-      S.ra[l] = grp_corr<MAT>(sqdist(qa.x, qa.y, px[l], py[l]), c, al, bt, mt);
+      S.ra[l] = grp_corr<MAT>(sqdist(qa.x, qa.y, px[l], py[l]), gc);
   });
   if constexpr (R == 2) {  // row u + 16
     static_for<0, 32>([&](auto lc) {
       constexpr int l = decltype(lc)::value;
       S.rb[l] = l == u + 16 ? (inb ? c.diag : 1.0) : 0.0;
       if (l < u + 16 && inb)
-        S.rb[l] = grp_corr<MAT>(sqdist(qb.x, qb.y, px[l], py[l]), c, al, bt, mt);
+        S.rb[l] = grp_corr<MAT>(sqdist(qb.x, qb.y, px[l], py[l]), gc);
     });
   }
   const double ca =
-      ina ? grp_corr<MAT>(sqdist(s.x, s.y, qa.x, qa.y), c, al, bt, mt) : 0.0;
+      ina ? grp_corr<MAT>(sqdist(s.x, s.y, qa.x, qa.y), gc) : 0.0;
   const double cb =
-      inb ? grp_corr<MAT>(sqdist(s.x, s.y, qb.x, qb.y), c, al, bt, mt) : 0.0;
+      inb ? grp_corr<MAT>(sqdist(s.x, s.y, qb.x, qb.y), gc) : 0.0;
   wave_sync();  // the row's coordinates are read; the next site rewrites them
   grp_in_ids<R>(P, u, in2);  // next site, stage 2
   bool ok = grp_factor<MM>(S, u);
@@ -1290,7 +1343,7 @@ template <int MM, bool MAT>
 __global__ __launch_bounds__(64 * kCoopMaxWaves) void k_bf_grp(BfArgs A) {
   extern __shared__ double smem[];
   __shared__ double red[kGrpSlots][kStatsMax];
-  __shared__ CoopTabs<false> tabs;
+  __shared__ double2 tab[MAT ? kMpLen / 2 : 1];
   __shared__ CovArgs cl;  // for the out-of-line matern series
   const int nw = (int)blockDim.x >> 6;
   const int w = (int)threadIdx.x >> 6;
@@ -1301,13 +1354,15 @@ __global__ __launch_bounds__(64 * kCoopMaxWaves) void k_bf_grp(BfArgs A) {
   if (b < 0) return;
   const BfProblem P = bf_problem<false>(A);
   const CovArgs c = A.c;
-  if (MAT) {  // the block's Bessel-K divisors and the pass's table
+  if (MAT) {  // the pass's table
     if (threadIdx.x == 0) cl = c;
-    bessel_tab_fill(tabs.bt, c);
+    const double2 *src = reinterpret_cast<const double2 *>(A.mtab);
+    for (int k = (int)threadIdx.x; k < kMpLen / 2; k += (int)blockDim.x)
+      tab[k] = src[k];
     __syncthreads();
-    matern_tab_fill(tabs.mt, c, tabs.bt, smem);
-    __syncthreads();  // its scratch becomes the waves' coordinate areas
   }
+  const GrpCov gc{c, cl, reinterpret_cast<const double *>(tab),
+                  *reinterpret_cast<const BesselTab *>(A.mtab + kMpLen)};
   double *px = smem + (size_t)w * grp_wave_doubles(MM) + (size_t)g * 2 * MM;
   double *py = px + MM;
   const int slot = 4 * w + g;
@@ -1331,8 +1386,7 @@ __global__ __launch_bounds__(64 * kCoopMaxWaves) void k_bf_grp(BfArgs A) {
     const bool valid2 = q2 < run.end && i2 < A.n;
     double F, e[kMaxNZ];
     GrpIn in2;
-    const bool ok = grp_site<MM, MAT>(A, P, c, cl, tabs.bt, tabs.mt, px, py,
-                                      i, valid, in, i2, valid2, in2, u, F, e);
+    const bool ok = grp_site<MM, MAT>(A, P, gc, px, py, i, valid, in, i2, valid2, in2, u, F, e);
     in = in2;
     if (valid && u == 0) {
       if (A.F) A.F[i] = F;
@@ -1496,7 +1550,8 @@ int bf_rows(const BfArgs &a, const BfConfig &cfg) {
   // the row kernel's waves take groups of four sites
   const int units = cfg.family == 2 ? (a.n + 3) / 4 : a.n;
   const int need = (units + waves - 1) / waves;
-  return need < kCoopBlocks ? need : kCoopBlocks;
+  const int most = cfg.family == 2 ? kGrpWaves / waves : kCoopBlocks;
+  return need < most ? need : most;
 }
 
 template <int M, bool BATCH>
@@ -1688,21 +1743,17 @@ static void launch_coop(const BfArgs &a, const dim3 &grid, const dim3 &blk,
   }
 }
 
-// LDS of the row kernel's block: the matern table's build, then the
-// waves' coordinate areas.
-static size_t grp_shm(const BfArgs &a, int waves, int mm) {
-  const size_t d = (size_t)waves * grp_wave_doubles(mm);
-  const size_t need =
-      a.c.cov == 2 && d < (size_t)kMatScratch ? (size_t)kMatScratch : d;
-  return need * sizeof(double);
-}
-
-static void launch_grp(const BfArgs &a, const dim3 &grid, const dim3 &blk,
-                       hipStream_t st) {
+static int launch_grp(const BfArgs &a, const dim3 &grid, const dim3 &blk,
+                      hipStream_t st) {
   const int waves = (int)blk.x / 64;
   const int mm = a.m <= 16 ? 16 : 32;
-  const size_t shm = grp_shm(a, waves, mm);
+  const size_t shm = (size_t)waves * grp_wave_doubles(mm) * sizeof(double);
   const bool mat = a.c.cov == 2;
+  if (mat) {
+    if (!a.mtab) return -2;
+    hipLaunchKernelGGL(k_matern_pieces, dim3(kMpOct), dim3(kMpThreads), 0, st,
+                       a.c, a.mtab);
+  }
   if (mm == 16) {
     if (mat) hipLaunchKernelGGL((k_bf_grp<16, true>), grid, blk, shm, st, a);
     else hipLaunchKernelGGL((k_bf_grp<16, false>), grid, blk, shm, st, a);
@@ -1710,6 +1761,7 @@ static void launch_grp(const BfArgs &a, const dim3 &grid, const dim3 &blk,
     if (mat) hipLaunchKernelGGL((k_bf_grp<32, true>), grid, blk, shm, st, a);
     else hipLaunchKernelGGL((k_bf_grp<32, false>), grid, blk, shm, st, a);
   }
+  return 0;
 }
 
 int bf_launch(const BfArgs &a0, const BfConfig &cfg, int nprob,
@@ -1738,7 +1790,7 @@ int bf_launch(const BfArgs &a0, const BfConfig &cfg, int nprob,
   } else if (cfg.family == 2) {
     if (batch || a.mixed) return -1;  // single FP64 problems only
     a.coop_blocks = nrows;
-    launch_grp(a, grid, blk, st);
+    if (const int rc = launch_grp(a, grid, blk, st)) return rc;
   } else {
     a.coop_blocks = nrows;
     const int waves = cfg.threads / 64;

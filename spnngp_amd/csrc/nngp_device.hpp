@@ -459,6 +459,49 @@ __device__ __forceinline__ double matern_s2_fast(double d, const CovArgs &a,
   return matern_tab_at(x, o, T);
 }
 
+// ---------------------------------------------------------------------------
+// the general-nu matern as a table in device memory (the row kernel)
+// ---------------------------------------------------------------------------
+// The same function on the same range [2^-30, 2^6) with each octave cut into
+// 16 equal pieces of the mantissa: the centre of a piece is at least 33
+// half-widths from the singularity at 0, so the interpolant at 9 Chebyshev
+// points (degree 8) converges like 66^-9 = 4e-17.  Nine coefficients an
+// entry instead of 16 matter because the row kernel is bound by its LDS
+// reads of them; the piece number is the exponent and the top four mantissa
+// bits of x, and a row of nine doubles puts neighboring pieces' k-th
+// coefficients in different LDS banks.  One small launch per pass fills the
+// table (k_matern_pieces); every block then copies it to LDS, instead of
+// evaluating the series at 1,152 nodes itself.
+constexpr int kMpOct0 = -30, kMpOct = 36;
+constexpr int kMpSub = 16;                 // pieces an octave
+constexpr int kMpN = 9;                    // coefficients a piece
+constexpr int kMpRows = kMpOct * kMpSub;
+constexpr int kMpLen = kMpRows * kMpN;     // doubles of the table
+// device buffer of a pass's table: the pieces, then the Bessel-K divisors
+constexpr size_t kMpBytes = kMpLen * sizeof(double) + sizeof(BesselTab);
+
+// Piece of x > 0; kMpRows or above (unsigned) outside the table, x <= 0,
+// infinities and NaN included.
+__device__ __forceinline__ unsigned matern_piece(double x) {
+  return ((unsigned)__double2hiint(x) >> 16) -
+         (unsigned)((1023 + kMpOct0) * kMpSub);
+}
+
+// The table's s2 * rho at x in piece r: the polynomial in m - c, m the
+// mantissa in [1, 2) and c the piece's centre (the difference is exact).
+__device__ __forceinline__ double matern_piece_at(double x, unsigned r,
+                                                  const double *T) {
+  const int hi = __double2hiint(x);
+  const double m = __hiloint2double((hi & 0xFFFFF) | 0x3FF00000,
+                                    __double2loint(x));
+  const double v = m - __hiloint2double((hi & 0xF0000) | 0x3FF08000, 0);
+  const double *p = T + r * kMpN;
+  double q = p[kMpN - 1];
+#pragma unroll
+  for (int k = kMpN - 2; k >= 0; k--) q = fma(q, v, p[k]);
+  return q;
+}
+
 // Covariance variants of the templated kernels: the four covModels, plus
 // the matern at nu = 1.5 and nu = 2.5 in closed form, (1 + x) e^-x and
 // (1 + x + x^2/3) e^-x with x = phi D (the Bessel-K expression of

@@ -287,6 +287,7 @@ int Model::create(int n_, int m_, int p_, const double *coords,
   }
   for (int s = 0; s < 2; s++) NNGP_TRY(F[s].alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(rows.alloc(sizeof(double) * (size_t)rows_capacity(n) * kStatsMax));
+  if (cov == 2) NNGP_TRY(mtab.alloc(kMpBytes));
   NNGP_TRY(sums.alloc(sizeof(double) * kSumsLen));
   NNGP_TRY(err.alloc(sizeof(int)));
   if (fill_int_launch(err.as<int>(), INT_MAX, st.s))
@@ -333,6 +334,7 @@ int Model::bf(const CovArgs &c, int slot, bool storeB) {
   a.variant = cov_variant(c.cov, c.nu);
   a.mixed = precision == NNGP_MIXED ? 1 : 0;
   a.lu_closed = lu_closed ? 1 : 0;
+  a.mtab = mtab.as<double>();
   BfConfig cfg = bf_default(m, a.variant, !a.mixed);
   if (a.mixed) {  // untuned mixed passes keep the covariance copy in
                   // registers (the fastest per-lane mixed shape at m = 15)
@@ -389,6 +391,7 @@ int Model::autotune(const CovArgs &c, BfTuneReport *rep) {
   a.variant = cov_variant(c.cov, c.nu);
   a.mixed = precision == NNGP_MIXED ? 1 : 0;
   a.lu_closed = lu_closed ? 1 : 0;
+  a.mtab = mtab.as<double>();
   BfConfig best;
   const int rc = bf_autotune(a, 1, st.s, &best, rep);
   if (rc) return set_err(NNGP_ERR_HIP, "autotune launch failed (%d)", rc);

@@ -285,6 +285,7 @@ struct Model {
   // sums: [0, kStatsMax) pass at off 0, [kStatsMax, 2 kStatsMax) pass at
   // off kStatsMax, then the updateBF failure flag of each (as doubles)
   DevBuf rows, sums, err;
+  DevBuf mtab;         // matern models: the row kernel's table (BfArgs::mtab)
   PinnedBuf hsums;  // host mirror of sums, then the completion word
   double *sums_mapped = nullptr;  // device address of hsums: the sum kernel
                                   // writes there directly (no copy)

@@ -46,6 +46,10 @@ struct BfArgs {
   // i(i-1)/2 for i < m, else m(m-1)/2 + (i-m)m; count min(i, m)), checked
   // on the host, so the per-lane kernel computes it instead of loading it
   int lu_closed = 0;
+  // kMpBytes of device memory for the pass's matern table: required by the
+  // row kernel when c.cov == 2, which fills it before its own launch (so
+  // passes that share it have to be on one stream)
+  double *mtab = nullptr;
 };
 
 // Offset and count of site i in the flat neighbor arrays when they follow
