@@ -41,777 +41,13 @@
 #include <tuple>
 #include <vector>
 
-#include "nngp_kernels.hpp"
-#include "nngp_group.hpp"
-#include "nngp_wave.hpp"
+#include "nngp_bf.hpp"
 
 namespace nngp {
-
-constexpr int kLaneMaxThreads = 256;
-constexpr int kCoopMaxWaves = 4;
-constexpr int kCoopMaxM = 64;
-constexpr int kCoopBlocks = 2048;  // logical blocks of the wavefront kernel
-constexpr int kGrpMaxM = 32;       // the row kernel's largest system
-// Waves of the row kernel: two a SIMD on 256 CUs, which is what its registers
-// allow, so that every block is resident and reads the matern table once.
-constexpr int kGrpWaves = 2048;
-constexpr int kRedThreads = 256;   // threads per block of the sum kernels
-constexpr int kRowsThreads = 1024; // threads per column of k_rows_sum
-constexpr int kRedBlocks = 1024;   // grid of the sum kernels (at most)
-
-// DPP lane move of a double (two 32-bit moves); lanes outside ROWMASK get 0.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ double dpp_mov(double v) {
-  const int lo = __builtin_amdgcn_update_dpp(0, __double2loint(v), CTRL,
-                                             ROWMASK, 0xF, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, __double2hiint(v), CTRL,
-                                             ROWMASK, 0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-// The same where lanes outside ROWMASK may receive anything (no value is
-// prepared for them): for sums whose result is read in lanes the move
-// reaches.
-template <int CTRL, int ROWMASK>
-__device__ __forceinline__ double dpp_mov_any(double v) {
-  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, ROWMASK,
-                                          0xF, false);
-  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, ROWMASK,
-                                          0xF, false);
-  return __hiloint2double(hi, lo);
-}
-
-// Sum over the 64 lanes with DPP moves only (no LDS round trips); the
-// total is valid in lane 63 (other lanes hold partial or meaningless
-// sums).  Fixed order: pairs, quads, half rows, rows, then rows 0+1 and
-// 2+3, then all four.
-__device__ __forceinline__ double wave_sum_to63(double x) {
-  x += dpp_mov_any<0xB1, 0xF>(x);   // quad_perm [1,0,3,2]
-  x += dpp_mov_any<0x4E, 0xF>(x);   // quad_perm [2,3,0,1]
-  x += dpp_mov_any<0x141, 0xF>(x);  // row_half_mirror
-  x += dpp_mov_any<0x140, 0xF>(x);  // row_mirror
-  x += dpp_mov_any<0x142, 0xA>(x);  // row_bcast:15 into rows 1 and 3
-  x += dpp_mov_any<0x143, 0xC>(x);  // row_bcast:31 into rows 2 and 3
-  return x;
-}
 
 int rows_capacity(int n) {
   const int lane_rows = (n + 63) / 64;  // smallest lane block is 64 threads
   return lane_rows > kCoopBlocks ? lane_rows : kCoopBlocks;
-}
-
-// ---------------------------------------------------------------------------
-// problem view
-// ---------------------------------------------------------------------------
-struct BfProblem {
-  const double2 *xy;
-  const int *nnIndx;
-  const int *lu;
-  const double *Z;
-  double *rows;
-  int *err;
-};
-
-template <bool BATCH>
-__device__ __forceinline__ BfProblem bf_problem(const BfArgs &A) {
-  BfProblem P{A.xy, A.nnIndx, A.lu, A.Z, A.rows, A.err};
-  if constexpr (BATCH) {
-    const int j = (int)blockIdx.y;
-    const int f = j / A.ng;
-    P.xy += (size_t)f * A.fs_xy;
-    P.nnIndx += (size_t)f * A.fs_nn;
-    P.lu += (size_t)f * A.fs_lu;
-    if (P.Z) P.Z += (size_t)f * A.fs_Z;
-    if (P.rows) P.rows += (size_t)j * A.ps_rows;
-    P.err += j;
-  }
-  return P;
-}
-
-// ---------------------------------------------------------------------------
-// one site per lane
-// ---------------------------------------------------------------------------
-
-// The block's partial row: column 0 sum log F_i, column 1 zero (quadratic
-// forms are formed from the cross-products), then the lower triangle of
-// e e^T / F row by row.  Called by every thread of the block.
-__device__ inline void block_site_terms(int nz, double *rows, int rows_cap,
-                                        bool valid, double F,
-                                        const double (&e)[kMaxNZ], int row) {
-  __shared__ double red[kLaneMaxThreads / 64][kStatsMax];
-  const int nw = (int)blockDim.x >> 6;
-  const int w = (int)threadIdx.x >> 6, t = (int)threadIdx.x & 63;
-  const double rf = valid ? 1.0 / F : 0.0;
-  double x = wave_sum_to63(valid ? log(F) : 0.0);
-  if (t == 63) red[w][0] = x;
-  int g = 2;
-#pragma unroll
-  for (int p = 0; p < kMaxNZ; p++) {
-    if (p < nz) {
-#pragma unroll
-      for (int q = 0; q <= p; q++) {
-        x = wave_sum_to63(e[p] * e[q] * rf);
-        if (t == 63) red[w][g + q] = x;
-      }
-    }
-    g += p + 1;
-  }
-  __syncthreads();
-  const int nv = 2 + nz * (nz + 1) / 2;
-  const int k = (int)threadIdx.x;
-  if (k < nv) {
-    double s = 0.0;
-    if (k != 1)
-      for (int ww = 0; ww < nw; ww++) s += red[ww][k];
-    rows[(size_t)k * rows_cap + row] = s;
-  }
-}
-
-// Number of per-site terms of a partial row (column 1, always 0, aside):
-// log F, then the nz(nz+1)/2 cross-products.
-__host__ __device__ constexpr int site_terms(int nz) {
-  return 1 + nz * (nz + 1) / 2;
-}
-
-// block_site_terms through LDS.  Each lane writes its terms to its wave's
-// area `w` (term v of lane t at w[v * 64 + t], site_terms(nz) x 64 doubles),
-// each quad of lanes then sums one term over 16 lanes apiece in lane order
-// and combines its four partials (pairs, then the two pairs), and with more
-// than one wave per block the wave sums meet in LDS and are added in wave
-// order.  The order is fixed, so a launch shape's sums are reproducible.
-// `w` may be memory the wave has finished reading (the staged covariate
-// rows); the barrier before the writes also keeps those reads first.
-__device__ inline void block_site_terms_lds(int nz, double *rows,
-                                            int rows_cap, bool valid,
-                                            double F,
-                                            const double (&e)[kMaxNZ],
-                                            int row, double *w) {
-  __shared__ double wsum[kLaneMaxThreads / 64][kStatsMax];
-  const int nw = (int)blockDim.x >> 6;
-  const int wv = (int)threadIdx.x >> 6, t = (int)threadIdx.x & 63;
-  const int nt = site_terms(nz);
-  const double rf = valid ? 1.0 / F : 0.0;
-  __syncthreads();
-  w[t] = valid ? log(F) : 0.0;
-  int g = 1;
-#pragma unroll
-  for (int p = 0; p < kMaxNZ; p++) {
-    if (p < nz) {
-#pragma unroll
-      for (int q = 0; q <= p; q++) w[(g + q) * 64 + t] = e[p] * e[q] * rf;
-    }
-    g += p + 1;
-  }
-  __syncthreads();
-  for (int v0 = 0; v0 < nt; v0 += 16) {
-    const int v = v0 + (t >> 2), qd = t & 3;
-    double s = 0.0;
-    if (v < nt) {
-      const double2 *src = reinterpret_cast<const double2 *>(w + v * 64 +
-                                                             qd * 16);
-#pragma unroll
-      for (int u = 0; u < 8; u++) {
-        const double2 x = src[u];
-        s += x.x;
-        s += x.y;
-      }
-    }
-    s += dpp_mov_any<0xB1, 0xF>(s);  // quad_perm [1,0,3,2]
-    s += dpp_mov_any<0x4E, 0xF>(s);  // quad_perm [2,3,0,1]
-    if (qd == 0 && v < nt) {
-      if (nw == 1)
-        rows[(size_t)(v == 0 ? 0 : v + 1) * rows_cap + row] = s;
-      else
-        wsum[wv][v] = s;
-    }
-  }
-  if (nw == 1) {
-    if (t == 0) rows[(size_t)rows_cap + row] = 0.0;
-    return;
-  }
-  __syncthreads();
-  const int k = (int)threadIdx.x;
-  if (k <= nt) {  // column k of the row: term k - 1 beyond column 1
-    double s = 0.0;
-    if (k != 1) {
-      const int v = k == 0 ? 0 : k - 1;
-      for (int ww = 0; ww < nw; ww++) s += wsum[ww][v];
-    }
-    rows[(size_t)k * rows_cap + row] = s;
-  }
-}
-
-// Direct-to-LDS load of 16 bytes a lane: lane t's bytes land at dst + t
-// (dst the same for the whole wavefront).  The load counts in vmcnt like any
-// other; the data are in LDS once it has been waited for.
-__device__ __forceinline__ void lds_load16(const double *src, double2 *dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void *)src,
-      (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-}
-
-// One site per lane: B_i, F_i and the residual vector e of site i from its
-// neighbor count, offset and index slots (slots past the count are not its
-// neighbors; they are replaced by site 0 here, before any use).
-// ZH > 0 stages the rows of Z (zs = 2 ZH doubles) of the M neighbor slots
-// and of the site itself in LDS with the coordinate gathers, instead of
-// gathering them into registers after the solve, where the wait for them
-// would stall the wavefront: chunk h of slot k (slot M = the site) at
-// stg[(k * ZH + h) * 64 + lane].  The residuals add the same terms in the
-// same order either way.
-template <int M, int COV, bool BATCH, int ZH = 0>
-__device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
-                                          const CovArgs &c, int i, int cnt,
-                                          int off, int (&nb)[M], double &Fi,
-                                          double (&e)[kMaxNZ],
-                                          double2 *stg = nullptr) {
-  if (cnt == 0) {  // site 0: F = s2 + t2, residual = the data
-    Fi = c.diag;
-#pragma unroll
-    for (int j = 0; j < kMaxNZ; j++)
-      if (j < A.nz) e[j] = P.Z[(size_t)i * A.zs + j];
-    return;
-  }
-  if (cnt < M) {
-#pragma unroll
-    for (int k = 0; k < M; k++)
-      if (k >= cnt) nb[k] = 0;
-  }
-  // The staged rows are requested before the coordinates: the hardware's
-  // load counter retires in order, so the one wait for the coordinates
-  // covers them too, and nothing waits on memory again until the residuals.
-  if constexpr (ZH > 0) {
-#pragma unroll
-    for (int k = 0; k <= M; k++) {
-      const double *zr = P.Z + (size_t)(k < M ? nb[k] : i) * (2 * ZH);
-#pragma unroll
-      for (int h = 0; h < ZH; h++)
-        lds_load16(zr + 2 * h, stg + (k * ZH + h) * 64);
-    }
-  }
-  // the site's own coordinates first, so that they arrive with the
-  // neighbors' (one wait for both)
-  const double2 s = P.xy[i];
-  double px[M], py[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    const double2 q = P.xy[nb[k]];
-    px[k] = q.x;
-    py[k] = q.y;
-  }
-  if (cnt < M) {
-#pragma unroll
-    for (int k = 0; k < M; k++) {
-      if (k >= cnt) {  // far away and far apart: zero correlation
-        px[k] = 1e100 * (k + 1);
-        py[k] = -1e100 * (k + 1);
-      }
-    }
-  }
-  // exponential, gaussian and the closed-form materns: neighbor offsets
-  // from the site, in units where the exponential factor is 2^-d (2^-d^2),
-  // see s2_exp2.  Offsetting first keeps large coordinate values (projected
-  // systems) out of the rounding of the scaled coordinates.
-  constexpr bool kBase2 = lane_base2<COV>();
-  if constexpr (kBase2) {
-#pragma unroll
-    for (int k = 0; k < M; k++) {
-      px[k] = (px[k] - s.x) * c.tsc;
-      py[k] = (py[k] - s.y) * c.tsc;
-    }
-  }
-
-  constexpr int T = M * (M + 1) / 2;
-  double a[T];  // packed lower triangle
-  double v[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    v[k] = lane_corr<COV>(kBase2 ? lane_d2<COV>(px[k], py[k])
-                                 : sqdist(s.x, s.y, px[k], py[k]),
-                          c);
-#pragma unroll
-    for (int l = 0; l < k; l++)
-      a[tri(k, l)] = lane_corr<COV>(
-          lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);
-    a[tri(k, k)] = c.diag;
-  }
-  double vv;
-  const bool ok = chol_solve<M>(a, v, vv);  // v <- B_i = C^-1 c
-  if (!BATCH && A.B) {
-#pragma unroll
-    for (int k = 0; k < M; k++)
-      if (k < cnt) A.B[off + k] = v[k];
-  }
-  Fi = c.diag - vv;
-  // residual vectors; padded coefficients are exactly 0
-  if constexpr (ZH > 0) {
-    const int t = (int)threadIdx.x & 63;
-#pragma unroll
-    for (int h = 0; h < ZH; h++) {
-      const double2 zi = stg[(M * ZH + h) * 64 + t];
-      double e0 = zi.x, e1 = zi.y;
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        const double2 z = stg[(k * ZH + h) * 64 + t];
-        e0 = fma(-v[k], z.x, e0);
-        e1 = fma(-v[k], z.y, e1);
-      }
-      e[2 * h] = e0;
-      e[2 * h + 1] = e1;
-    }
-    if (!ok) atomicMin(P.err, i);
-    return;
-  }
-#pragma unroll
-  for (int j = 0; j < kMaxNZ; j++) {
-    if (j < A.nz) {
-      double ej = P.Z[(size_t)i * A.zs + j];
-#pragma unroll
-      for (int k = 0; k < M; k++)
-        ej = fma(-v[k], P.Z[(size_t)nb[k] * A.zs + j], ej);
-      e[j] = ej;
-    }
-  }
-  if (!ok) atomicMin(P.err, i);
-}
-
-template <int M, int COV, bool BATCH>
-__global__ __launch_bounds__(kLaneMaxThreads) void k_bf_lane(BfArgs A) {
-  extern __shared__ double lane_red[];  // site_terms(nz) x 64 per wave
-  const int nt = (int)blockDim.x;
-  const int b = xcd_block((A.n + nt - 1) / nt);
-  if (b < 0) return;  // whole padding block
-  const BfProblem P = bf_problem<BATCH>(A);
-  const CovArgs c = BATCH ? A.covs[(int)blockIdx.y % A.ng] : A.c;
-  const int i = b * nt + (int)threadIdx.x;
-  const bool valid = i < A.n;
-  double Fi = 1.0;
-  double e[kMaxNZ];
-#pragma unroll
-  for (int j = 0; j < kMaxNZ; j++) e[j] = 0.0;
-
-  if (valid) {
-    int cnt, off;
-    if (A.lu_closed) {
-      nn_closed(i, A.m, off, cnt);
-    } else {
-      cnt = P.lu[A.n + i];
-      off = P.lu[i];
-    }
-    // The index array carries 64 padding entries, so off + k is in bounds.
-    int nb[M];
-#pragma unroll
-    for (int k = 0; k < M; k++) nb[k] = P.nnIndx[off + k];
-    lane_site<M, COV, BATCH>(A, P, c, i, cnt, off, nb, Fi, e);
-    if (!BATCH && A.F) A.F[i] = Fi;
-  }
-  if (P.rows) {
-    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-    block_site_terms_lds(A.nz, P.rows, A.rows_cap, valid, Fi, e, b,
-                         lane_red + (size_t)w * site_terms(A.nz) * 64);
-  }
-}
-
-// k_bf_lane with the covariate rows staged in LDS: the block's dynamic LDS
-// holds, per wavefront, (M + 1) x ZH chunks of 64 x 16 bytes.  The launcher
-// uses it only when Z is set, zs = 2 ZH and every problem's Z is 16-byte
-// aligned.
-template <int M, int COV, int ZH, bool BATCH>
-__global__ __launch_bounds__(kLaneMaxThreads) void k_bf_lane_lds(BfArgs A) {
-  extern __shared__ double2 zstage[];
-  const int nt = (int)blockDim.x;
-  const int b = xcd_block((A.n + nt - 1) / nt);
-  if (b < 0) return;  // whole padding block
-  const BfProblem P = bf_problem<BATCH>(A);
-  const CovArgs c = BATCH ? A.covs[(int)blockIdx.y % A.ng] : A.c;
-  const int i = b * nt + (int)threadIdx.x;
-  const bool valid = i < A.n;
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  double2 *stg = zstage + (size_t)w * (M + 1) * ZH * 64;
-  double Fi = 1.0;
-  double e[kMaxNZ];
-#pragma unroll
-  for (int j = 0; j < kMaxNZ; j++) e[j] = 0.0;
-
-  if (valid) {
-    int cnt, off;
-    if (A.lu_closed) {
-      nn_closed(i, A.m, off, cnt);
-    } else {
-      cnt = P.lu[A.n + i];
-      off = P.lu[i];
-    }
-    int nb[M];
-#pragma unroll
-    for (int k = 0; k < M; k++) nb[k] = P.nnIndx[off + k];
-    lane_site<M, COV, BATCH, ZH>(A, P, c, i, cnt, off, nb, Fi, e, stg);
-    if (!BATCH && A.F) A.F[i] = Fi;
-  }
-  // the sums reuse the wave's staging area (the residuals have read it);
-  // site_terms(nz) <= 11 doubles a lane fit in (M + 1) x ZH x 16 bytes
-  if (P.rows)
-    block_site_terms_lds(A.nz, P.rows, A.rows_cap, valid, Fi, e, b,
-                         reinterpret_cast<double *>(stg));
-}
-
-// ---------------------------------------------------------------------------
-// mixed precision, one site per lane
-// ---------------------------------------------------------------------------
-// The covariance is built in FP32 from FP32 neighbor offsets (FP64
-// differences to the site, rounded), factored and solved in FP32 for B0.
-// One refinement step forms the residual r = c - C B0 of that FP32 system
-// in FP64 arithmetic (each FP32 x FP64 product is exact before the sum),
-// solves C d = r with the FP32 factor and sets B = B0 + d, which removes
-// the factorization's error.  F = s2 + t2 - c.B and every sum stay in FP64.
-// What remains is the FP32 rounding of the covariance entries themselves.
-// COPY = true keeps C in LDS (lane-interleaved) for the residual; false
-// evaluates the entries a second time (bit-identically) to save LDS.
-template <int COV>
-__device__ __forceinline__ float pair32(float dxk, float dyk, float dxl,
-                                        float dyl, const CovArgs32 &c) {
-  const float ex = dxk - dxl, ey = dyk - dyl;
-  return s2_corr32<COV>(fmaf(ex, ex, ey * ey), c);
-}
-
-template <int M, int COV, bool COPY>
-__global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed(BfArgs A) {
-  // COPY: covariance entry t of lane L at cl[t*nt + L]; otherwise the
-  // neighbor offsets dx_k at cl[k*nt + L], dy_k at cl[(M+k)*nt + L]
-  extern __shared__ float cl[];
-  const int nt = (int)blockDim.x;
-  const int b = xcd_block((A.n + nt - 1) / nt);
-  if (b < 0) return;
-  const CovArgs &c = A.c;
-  const CovArgs32 c32 = cov32(c);
-  const int L = (int)threadIdx.x;
-  const int i = b * nt + L;
-  const bool valid = i < A.n;
-  double Fi = 1.0;
-  double e[kMaxNZ];  // set on every path just before use (no value is live
-                     // through the factorization)
-
-  if (valid) {
-    int cnt, off;
-    if (A.lu_closed) {
-      nn_closed(i, A.m, off, cnt);
-    } else {
-      cnt = A.lu[A.n + i];
-      off = A.lu[i];
-    }
-    if (cnt == 0) {
-      Fi = c.diag;
-#pragma unroll
-      for (int j = 0; j < kMaxNZ; j++)
-        e[j] = j < A.nz ? A.Z[(size_t)i * A.zs + j] : 0.0;
-    } else {
-      const double2 s = A.xy[i];
-      // as in k_bf_lane: padding entries of the index read as site 0, then
-      // replaced by far-away finite offsets (every product with one is +inf
-      // or 0 in FP32, so its correlations are exactly 0)
-      int nb[M];
-#pragma unroll
-      for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
-      if (cnt < M) {
-#pragma unroll
-        for (int k = 0; k < M; k++)
-          if (k >= cnt) nb[k] = 0;
-      }
-      float dx[M], dy[M];
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        const double2 q = A.xy[nb[k]];
-        dx[k] = (float)(q.x - s.x);
-        dy[k] = (float)(q.y - s.y);
-      }
-      if (cnt < M) {
-#pragma unroll
-        for (int k = 0; k < M; k++) {
-          if (k >= cnt) {
-            dx[k] = 1e30f * (k + 1);
-            dy[k] = -1e30f * (k + 1);
-          }
-        }
-      }
-      if (!COPY) {  // read back by the residual; registers stay free
-#pragma unroll
-        for (int k = 0; k < M; k++) {
-          cl[k * nt + L] = dx[k];
-          cl[(M + k) * nt + L] = dy[k];
-        }
-      }
-      constexpr int T = M * (M + 1) / 2;
-      float a[T], v[M];
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        if (COPY) {
-          v[k] = s2_corr32<COV>(fmaf(dx[k], dx[k], dy[k] * dy[k]), c32);
-          cl[(T + k) * nt + L] = v[k];
-        }
-#pragma unroll
-        for (int l = 0; l < k; l++) {
-          a[tri(k, l)] = pair32<COV>(dx[k], dy[k], dx[l], dy[l], c32);
-          if (COPY) cl[tri(k, l) * nt + L] = a[tri(k, l)];
-        }
-        a[tri(k, k)] = c32.diag;
-      }
-      const bool ok = chol_factor32<M>(a);
-      if (!COPY) {  // c after the factorization, from the offsets in LDS
-#pragma unroll
-        for (int k = 0; k < M; k++) {
-          const float xk = cl[k * nt + L], yk = cl[(M + k) * nt + L];
-          v[k] = s2_corr32<COV>(fmaf(xk, xk, yk * yk), c32);
-        }
-      }
-      chol_apply32<M>(a, v);  // v <- B0
-      // residual r = c - C B0 in FP64; B0 stays FP32 (converted where
-      // used), so only r is an FP64 array while the factor is live
-      double r[M];
-      const double dg = (double)c32.diag;
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        float ck;
-        if (COPY) {
-          ck = cl[(T + k) * nt + L];
-        } else {
-          const float xk = cl[k * nt + L], yk = cl[(M + k) * nt + L];
-          ck = s2_corr32<COV>(fmaf(xk, xk, yk * yk), c32);
-        }
-        r[k] = fma(-dg, (double)v[k], (double)ck);
-      }
-#pragma unroll
-      for (int k = 1; k < M; k++) {
-        float xk = 0.0f, yk = 0.0f;
-        if (!COPY) {
-          xk = cl[k * nt + L];
-          yk = cl[(M + k) * nt + L];
-        }
-#pragma unroll
-        for (int l = 0; l < k; l++) {
-          const double ckl =
-              COPY ? (double)cl[tri(k, l) * nt + L]
-                   : (double)pair32<COV>(xk, yk, cl[l * nt + L],
-                                         cl[(M + l) * nt + L], c32);
-          r[k] = fma(-ckl, (double)v[l], r[k]);
-          r[l] = fma(-ckl, (double)v[k], r[l]);
-        }
-      }
-      float d[M];
-#pragma unroll
-      for (int k = 0; k < M; k++) d[k] = (float)r[k];
-      chol_apply32<M>(a, d);  // d <- C^-1 r
-      double bd[M];
-      double cb = 0.0;
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        bd[k] = (double)v[k] + (double)d[k];
-        float ck;
-        if (COPY) {
-          ck = cl[(T + k) * nt + L];
-        } else {
-          const float xk = cl[k * nt + L], yk = cl[(M + k) * nt + L];
-          ck = s2_corr32<COV>(fmaf(xk, xk, yk * yk), c32);
-        }
-        cb = fma((double)ck, bd[k], cb);
-      }
-      if (A.B) {
-#pragma unroll
-        for (int k = 0; k < M; k++)
-          if (k < cnt) A.B[off + k] = bd[k];
-      }
-      Fi = c.diag - cb;
-      // the neighbor slots again (cache hits) rather than held in
-      // registers through the factorization; padded coefficients are 0
-#pragma unroll
-      for (int k = 0; k < M; k++) nb[k] = k < cnt ? A.nnIndx[off + k] : 0;
-#pragma unroll
-      for (int j = 0; j < kMaxNZ; j++) {
-        e[j] = 0.0;
-        if (j < A.nz) {
-          double ej = A.Z[(size_t)i * A.zs + j];
-#pragma unroll
-          for (int k = 0; k < M; k++)
-            ej = fma(-bd[k], A.Z[(size_t)nb[k] * A.zs + j], ej);
-          e[j] = ej;
-        }
-      }
-      if (!ok || !(Fi > 0.0)) atomicMin(A.err, i);
-    }
-    if (A.F) A.F[i] = Fi;
-  } else {
-#pragma unroll
-    for (int j = 0; j < kMaxNZ; j++) e[j] = 0.0;
-  }
-  if (A.rows) block_site_terms(A.nz, A.rows, A.rows_cap, valid, Fi, e, b);
-}
-
-// k_bf_mixed's scheme at one wave per SIMD, where the FP32 factor and a
-// register copy of C both fit: no entry is evaluated twice and C does not
-// go through LDS.  The arithmetic is k_bf_mixed's step for step, so B and F
-// equal its results bit for bit.  As in lane_site, ZH > 0 stages the
-// covariate rows of the M neighbor slots and of the site in LDS with the
-// coordinate gathers (chunk h of slot k at stg[(k * ZH + h) * 64 + lane]).
-template <int M, int COV, int ZH>
-__device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
-                                               int cnt, int off,
-                                               int (&nb)[M], double &Fi,
-                                               double (&e)[kMaxNZ],
-                                               double2 *stg) {
-  const CovArgs &c = A.c;
-  const CovArgs32 c32 = cov32(c);
-  if (cnt == 0) {  // site 0: F = s2 + t2, residual = the data
-    Fi = c.diag;
-#pragma unroll
-    for (int j = 0; j < kMaxNZ; j++)
-      if (j < A.nz) e[j] = A.Z[(size_t)i * A.zs + j];
-    return;
-  }
-  if (cnt < M) {
-#pragma unroll
-    for (int k = 0; k < M; k++)
-      if (k >= cnt) nb[k] = 0;
-  }
-  if constexpr (ZH > 0) {
-#pragma unroll
-    for (int k = 0; k <= M; k++) {
-      const double *zr = A.Z + (size_t)(k < M ? nb[k] : i) * (2 * ZH);
-#pragma unroll
-      for (int h = 0; h < ZH; h++)
-        lds_load16(zr + 2 * h, stg + (k * ZH + h) * 64);
-    }
-  }
-  const double2 s = A.xy[i];
-  float dx[M], dy[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    const double2 q = A.xy[nb[k]];
-    dx[k] = (float)(q.x - s.x);
-    dy[k] = (float)(q.y - s.y);
-  }
-  if (cnt < M) {  // far away and far apart: correlations exactly 0
-#pragma unroll
-    for (int k = 0; k < M; k++) {
-      if (k >= cnt) {
-        dx[k] = 1e30f * (k + 1);
-        dy[k] = -1e30f * (k + 1);
-      }
-    }
-  }
-  constexpr int T = M * (M + 1) / 2;
-  float a[T], ac[T], v[M], cv[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    v[k] = s2_corr32<COV>(fmaf(dx[k], dx[k], dy[k] * dy[k]), c32);
-    cv[k] = v[k];
-#pragma unroll
-    for (int l = 0; l < k; l++) {
-      a[tri(k, l)] = pair32<COV>(dx[k], dy[k], dx[l], dy[l], c32);
-      ac[tri(k, l)] = a[tri(k, l)];
-    }
-    a[tri(k, k)] = c32.diag;
-  }
-  const bool ok = chol_factor32<M>(a);
-  chol_apply32<M>(a, v);  // v <- B0
-  // residual r = c - C B0 in FP64
-  double r[M];
-  const double dg = (double)c32.diag;
-#pragma unroll
-  for (int k = 0; k < M; k++) r[k] = fma(-dg, (double)v[k], (double)cv[k]);
-#pragma unroll
-  for (int k = 1; k < M; k++) {
-#pragma unroll
-    for (int l = 0; l < k; l++) {
-      const double ckl = (double)ac[tri(k, l)];
-      r[k] = fma(-ckl, (double)v[l], r[k]);
-      r[l] = fma(-ckl, (double)v[k], r[l]);
-    }
-  }
-  float d[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) d[k] = (float)r[k];
-  chol_apply32<M>(a, d);  // d <- C^-1 r
-  double bd[M];
-  double cb = 0.0;
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    bd[k] = (double)v[k] + (double)d[k];
-    cb = fma((double)cv[k], bd[k], cb);
-  }
-  if (A.B) {
-#pragma unroll
-    for (int k = 0; k < M; k++)
-      if (k < cnt) A.B[off + k] = bd[k];
-  }
-  Fi = c.diag - cb;
-  // residual vectors; padded coefficients are 0
-  if constexpr (ZH > 0) {
-    const int t = (int)threadIdx.x & 63;
-#pragma unroll
-    for (int h = 0; h < ZH; h++) {
-      const double2 zi = stg[(M * ZH + h) * 64 + t];
-      double e0 = zi.x, e1 = zi.y;
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        const double2 z = stg[(k * ZH + h) * 64 + t];
-        e0 = fma(-bd[k], z.x, e0);
-        e1 = fma(-bd[k], z.y, e1);
-      }
-      e[2 * h] = e0;
-      e[2 * h + 1] = e1;
-    }
-  } else {
-#pragma unroll
-    for (int j = 0; j < kMaxNZ; j++) {
-      if (j < A.nz) {
-        double ej = A.Z[(size_t)i * A.zs + j];
-#pragma unroll
-        for (int k = 0; k < M; k++)
-          ej = fma(-bd[k], A.Z[(size_t)nb[k] * A.zs + j], ej);
-        e[j] = ej;
-      }
-    }
-  }
-  if (!ok || !(Fi > 0.0)) atomicMin(A.err, i);
-}
-
-// Dynamic LDS of k_bf_mixed_reg a wavefront, in double2: the staged rows,
-// which the block sums then reuse, or the sums' area alone.
-__host__ __device__ inline int mixed_reg_wave_chunks(int M, int ZH, int nz) {
-  const int sums = (site_terms(nz) * 64 + 1) / 2;
-  const int stage = (M + 1) * ZH * 64;
-  return stage > sums ? stage : sums;
-}
-
-template <int M, int COV, int ZH>
-__global__ __launch_bounds__(kLaneMaxThreads) void k_bf_mixed_reg(BfArgs A) {
-  extern __shared__ double2 mstage[];
-  const int nt = (int)blockDim.x;
-  const int b = xcd_block((A.n + nt - 1) / nt);
-  if (b < 0) return;  // whole padding block
-  const int i = b * nt + (int)threadIdx.x;
-  const bool valid = i < A.n;
-  const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  double2 *stg = mstage + (size_t)w * mixed_reg_wave_chunks(M, ZH, A.nz);
-  double Fi = 1.0;
-  double e[kMaxNZ];
-#pragma unroll
-  for (int j = 0; j < kMaxNZ; j++) e[j] = 0.0;
-  if (valid) {
-    int cnt, off;
-    if (A.lu_closed) {
-      nn_closed(i, A.m, off, cnt);
-    } else {
-      cnt = A.lu[A.n + i];
-      off = A.lu[i];
-    }
-    int nb[M];
-#pragma unroll
-    for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
-    mixed_reg_site<M, COV, ZH>(A, i, cnt, off, nb, Fi, e, stg);
-    if (A.F) A.F[i] = Fi;
-  }
-  if (A.rows)
-    block_site_terms_lds(A.nz, A.rows, A.rows_cap, valid, Fi, e, b,
-                         reinterpret_cast<double *>(stg));
 }
 
 // ---------------------------------------------------------------------------
@@ -1119,304 +355,6 @@ __global__ __launch_bounds__(64 * kCoopMaxWaves) void k_bf_coop(BfArgs A) {
 }
 
 // ---------------------------------------------------------------------------
-// one site per 16-lane row (four sites per wavefront), m <= 32
-// ---------------------------------------------------------------------------
-constexpr int kGrpSlots = 4 * kCoopMaxWaves;  // sites a block works on at once
-
-// Per-wave LDS of the row kernel, in doubles: each of its four rows'
-// neighbor coordinates, x then y.
-__host__ __device__ inline int grp_wave_doubles(int mm) { return 4 * 2 * mm; }
-
-// The pass's matern table (matern_piece): block o fills the pieces of octave
-// o from the series at their Chebyshev points; block 0 also writes the
-// Bessel-K loop divisors behind the table, for the entries outside it.
-// 36 blocks take about as long as one series evaluation; with every block of
-// the row kernel building a table for itself (and 16 coefficients an entry) a
-// pass took 261 us at n = 1e5, m = 15 and 1.99 ms at n = 5e5, m = 32; with
-// this launch before it, 140 us and 1.53 ms.
-constexpr int kMpThreads = 192;  // at least kMpSub * kMpN
-
-__global__ __launch_bounds__(kMpThreads) void k_matern_pieces(CovArgs c,
-                                                              double *out) {
-  __shared__ BesselTab bt;
-  __shared__ double fv[kMpSub * kMpN], cc[kMpSub * kMpN];
-  bessel_tab_fill(bt, c);
-  __syncthreads();
-  const int q = (int)threadIdx.x, o = (int)blockIdx.x;
-  const int pc = q / kMpN, j = q % kMpN;  // piece of the octave, node
-  if (q < kMpSub * kMpN) {
-    const double u = cospi((j + 0.5) / kMpN);
-    const double m = 1.0 + (pc + 0.5 + 0.5 * u) / kMpSub;
-    fv[q] = c.mnorm * xnu_bessel_k(ldexp(m, kMpOct0 + o), c, bt);
-  }
-  __syncthreads();
-  if (q < kMpSub * kMpN) {  // Chebyshev coefficient j of the piece
-    double s = 0.0;
-    for (int k = 0; k < kMpN; k++)
-      s = fma(fv[pc * kMpN + k], cospi(j * (k + 0.5) / kMpN), s);
-    cc[q] = s * (j == 0 ? 1.0 / kMpN : 2.0 / kMpN);
-  }
-  __syncthreads();
-  if (q < kMpSub * kMpN) {  // coefficient of (m - c)^j, u = 2 kMpSub (m - c)
-    double s = 0.0;
-    for (int k = j; k < kMpN; k++)
-      s = fma(cc[pc * kMpN + k], kChebMono.t[k][j], s);
-    out[(o * kMpSub + pc) * kMpN + j] = s * ldexp(1.0, 5 * j);
-  }
-  if (o == 0) {
-    const double *src = reinterpret_cast<const double *>(&bt);
-    for (int k = q; k < (int)(sizeof(BesselTab) / sizeof(double));
-         k += kMpThreads)
-      out[kMpLen + k] = src[k];
-  }
-}
-static_assert(2 * kMpSub == 32, "u = 2^5 (m - c)");
-
-// Covariance entries of the row kernel.  A lane evaluates about fifty per
-// site in fully unrolled code, so only the common path is inline: for the
-// matern (MAT) the pass's table, with coincident or nearly coincident sites
-// and x >= 64 (outside the table) out of line; otherwise the exponential,
-// spherical and gaussian.  The out-of-line series reads the parameters from
-// the block's LDS copy `al` (a reference to the kernel argument would make
-// the kernel keep a stack copy of it and read the inline path's fields from
-// there).
-__device__ __noinline__ double grp_matern_outside(double x, const CovArgs &al,
-                                                  const BesselTab &bt) {
-  if (!(x > 0.0)) return al.s2;
-  if (x > 700.0) return 0.0;
-  return al.mnorm * xnu_bessel_k(x, al, bt);
-}
-
-// Where the row kernel's entries come from: the parameters and, for the
-// matern, their LDS copy, the table (LDS) and the divisors (device memory).
-struct GrpCov {
-  const CovArgs &a, &al;
-  const double *T;
-  const BesselTab &bt;
-};
-
-template <bool MAT>
-__device__ __forceinline__ double grp_corr(double d2, const GrpCov &c) {
-  if constexpr (MAT) {
-    const double x = nn_sqrt(d2) * c.a.phi;
-    const unsigned r = matern_piece(x);
-    if (r >= (unsigned)kMpRows) return grp_matern_outside(x, c.al, c.bt);
-    return matern_piece_at(x, r, c.T);
-  } else {
-    switch (c.a.cov) {
-      case 0: return s2_corr<0>(d2, c.a);
-      case 1: return s2_corr<1>(d2, c.a);
-      default: return s2_corr<3>(d2, c.a);
-    }
-  }
-}
-
-// A site's inputs on its row: neighbor count and offset, the lane's two
-// neighbor ids and coordinates, the site's coordinates.  The three loads
-// depend on each other, so the row kernel fetches the next site's in three
-// stages spread over the current site's work.
-struct GrpIn {
-  int cnt, off, ida, idb;
-  double2 qa, qb, s;
-};
-
-__device__ __forceinline__ void grp_in_lu(const BfArgs &A, const BfProblem &P,
-                                          int i, bool valid, GrpIn &in) {
-  in.cnt = 0;
-  in.off = 0;
-  if (valid) {
-    in.cnt = P.lu[A.n + i];
-    in.off = P.lu[i];
-  }
-}
-
-template <int R>
-__device__ __forceinline__ void grp_in_ids(const BfProblem &P, int u,
-                                           GrpIn &in) {
-  in.ida = 0;
-  in.idb = 0;
-  if (u < in.cnt) in.ida = P.nnIndx[in.off + u];
-  if (R == 2 && u + 16 < in.cnt) in.idb = P.nnIndx[in.off + u + 16];
-}
-
-template <int R>
-__device__ __forceinline__ void grp_in_xy(const BfProblem &P, int u, int i,
-                                          bool valid, GrpIn &in) {
-  in.qa = make_double2(0.0, 0.0);
-  in.qb = in.qa;
-  in.s = in.qa;
-  if (u < in.cnt) in.qa = P.xy[in.ida];
-  if (R == 2 && u + 16 < in.cnt) in.qb = P.xy[in.idb];
-  if (valid) in.s = P.xy[i];
-}
-
-// Site i on the 16-lane row of lane u (valid: i < n), its inputs in `in`.
-// The lane builds rows u and u + 16 of the site's system in registers from
-// the neighbor coordinates the row stages in px/py (rows past the site's
-// count are identity rows with a zero right-hand side, so B and F are those
-// of the cnt x cnt system), then factor, forward and back substitution
-// (nngp_group.hpp).  Meanwhile it fetches the inputs of the row's next site
-// in2 (site i2, valid2).  Every lane of the row returns F and the residuals
-// e; false when a pivot or F is not positive.
-template <int MM, bool MAT>
-__device__ inline bool grp_site(const BfArgs &A, const BfProblem &P,
-                                const GrpCov &gc, double *px, double *py,
-                                int i, bool valid, const GrpIn &in, int i2,
-                                bool valid2, GrpIn &in2, int u, double &F,
-                                double (&e)[kMaxNZ]) {
-  constexpr int R = GrpRows<MM>::R;
-  // opaque per site: the compares of u with every row number below would
-  // otherwise be hoisted out of the caller's site loop as lane masks, more
-  // than the SGPR file holds
-  u = lane_opaque(u);
-  const CovArgs &c = gc.a;
-  const int cnt = in.cnt, off = in.off, ida = in.ida, idb = in.idb;
-  const double2 qa = in.qa, qb = in.qb, s = in.s;
-  const bool ina = u < cnt, inb = R == 2 && u + 16 < cnt;
-  grp_in_lu(A, P, i2, valid2, in2);  // next site, stage 1
-  px[u] = qa.x;
-  py[u] = qa.y;
-  if constexpr (R == 2) {
-    px[u + 16] = qb.x;
-    py[u + 16] = qb.y;
-  }
-  wave_sync();
-  GrpRows<MM> S;
-  // row u: entries l < u, the diagonal, zeros above it
-  static_for<0, 16>([&](auto lc) {
-    constexpr int l = decltype(lc)::value;
-    S.ra[l] = l == u ? (ina ? c.diag : 1.0) : 0.0;
-    if (l < u && ina)
-      S.ra[l] = grp_corr<MAT>(sqdist(qa.x, qa.y, px[l], py[l]), gc);
-  });
-  if constexpr (R == 2) {  // row u + 16
-    static_for<0, 32>([&](auto lc) {
-      constexpr int l = decltype(lc)::value;
-      S.rb[l] = l == u + 16 ? (inb ? c.diag : 1.0) : 0.0;
-      if (l < u + 16 && inb)
-        S.rb[l] = grp_corr<MAT>(sqdist(qb.x, qb.y, px[l], py[l]), gc);
-    });
-  }
-  const double ca =
-      ina ? grp_corr<MAT>(sqdist(s.x, s.y, qa.x, qa.y), gc) : 0.0;
-  const double cb =
-      inb ? grp_corr<MAT>(sqdist(s.x, s.y, qb.x, qb.y), gc) : 0.0;
-  wave_sync();  // the row's coordinates are read; the next site rewrites them
-  grp_in_ids<R>(P, u, in2);  // next site, stage 2
-  bool ok = grp_factor<MM>(S, u);
-  grp_in_xy<R>(P, u, i2, valid2, in2);  // next site, stage 3
-  double ya, yb, ba, bb;
-  grp_forward<MM>(S, u, ca, cb, ya, yb);
-  F = c.diag - row_sum16(ya * ya + yb * yb);
-  grp_backward<MM>(S, u, ya, yb, ba, bb);
-  ok = ok && F > 0.0;
-  if (valid && A.B) {
-    if (ina) A.B[off + u] = ba;
-    if (inb) A.B[off + u + 16] = bb;
-  }
-#pragma unroll
-  for (int j = 0; j < kMaxNZ; j++) {
-    e[j] = 0.0;
-    if (j < A.nz) {
-      double part = 0.0;
-      if (ina) part = ba * P.Z[(size_t)ida * A.zs + j];
-      if (inb) part = fma(bb, P.Z[(size_t)idb * A.zs + j], part);
-      part = row_sum16(part);
-      e[j] = valid ? P.Z[(size_t)i * A.zs + j] - part : 0.0;
-    }
-  }
-  if (!ok) {
-    F = 1.0;  // keeps the sums finite; the pass reports the failure
-#pragma unroll
-    for (int j = 0; j < kMaxNZ; j++) e[j] = 0.0;
-  }
-  return ok;
-}
-
-// Logical block b (xcd_block) takes groups of four consecutive sites from
-// its XCD's run (xcd_site_run over the groups); each wave works on one
-// group, row g of the wave on site 4 q + g.  Each row's running sums live
-// in its own LDS slot (lane 0 of the row updates them); the block's row of
-// partial sums adds the slots in a fixed order.  Single problem, FP64.
-// MAT: the matern (c.cov == 2), by the pass's table.
-template <int MM, bool MAT>
-__global__ __launch_bounds__(64 * kCoopMaxWaves) void k_bf_grp(BfArgs A) {
-  extern __shared__ double smem[];
-  __shared__ double red[kGrpSlots][kStatsMax];
-  __shared__ double2 tab[MAT ? kMpLen / 2 : 1];
-  __shared__ CovArgs cl;  // for the out-of-line matern series
-  const int nw = (int)blockDim.x >> 6;
-  const int w = (int)threadIdx.x >> 6;
-  const int t = (int)threadIdx.x & 63;
-  const int g = t >> 4;
-  const int u = t & 15;
-  const int b = xcd_block(A.coop_blocks);
-  if (b < 0) return;
-  const BfProblem P = bf_problem<false>(A);
-  const CovArgs c = A.c;
-  if (MAT) {  // the pass's table
-    if (threadIdx.x == 0) cl = c;
-    const double2 *src = reinterpret_cast<const double2 *>(A.mtab);
-    for (int k = (int)threadIdx.x; k < kMpLen / 2; k += (int)blockDim.x)
-      tab[k] = src[k];
-    __syncthreads();
-  }
-  const GrpCov gc{c, cl, reinterpret_cast<const double *>(tab),
-                  *reinterpret_cast<const BesselTab *>(A.mtab + kMpLen)};
-  double *px = smem + (size_t)w * grp_wave_doubles(MM) + (size_t)g * 2 * MM;
-  double *py = px + MM;
-  const int slot = 4 * w + g;
-  const int nv = 2 + A.nz * (A.nz + 1) / 2;
-  for (int k = u; k < nv; k += 16) red[slot][k] = 0.0;
-  wave_sync();
-  const SiteRun run = xcd_site_run(A.coop_blocks, b, (A.n + 3) >> 2, nw, w);
-  GrpIn in;
-  {  // the first site's inputs; later sites' arrive during their
-     // predecessor's work
-    const int i = 4 * run.first + g;
-    const bool valid = run.first < run.end && i < A.n;
-    grp_in_lu(A, P, i, valid, in);
-    grp_in_ids<GrpRows<MM>::R>(P, u, in);
-    grp_in_xy<GrpRows<MM>::R>(P, u, i, valid, in);
-  }
-  for (int q = run.first; q < run.end; q += run.stride) {
-    const int i = 4 * q + g;
-    const bool valid = i < A.n;
-    const int q2 = q + run.stride, i2 = 4 * q2 + g;
-    const bool valid2 = q2 < run.end && i2 < A.n;
-    double F, e[kMaxNZ];
-    GrpIn in2;
-    const bool ok = grp_site<MM, MAT>(A, P, gc, px, py, i, valid, in, i2, valid2, in2, u, F, e);
-    in = in2;
-    if (valid && u == 0) {
-      if (A.F) A.F[i] = F;
-      if (!ok) atomicMin(P.err, i);
-      const double rf = 1.0 / F;
-      red[slot][0] += log(F);
-      int gg = 2;
-#pragma unroll
-      for (int p = 0; p < kMaxNZ; p++) {
-        if (p < A.nz) {
-#pragma unroll
-          for (int qq = 0; qq <= p; qq++)
-            red[slot][gg + qq] += e[p] * e[qq] * rf;
-        }
-        gg += p + 1;
-      }
-    }
-  }
-  if (!P.rows) return;
-  __syncthreads();
-  const int k = (int)threadIdx.x;
-  if (k < nv) {
-    double sum = 0.0;
-    if (k != 1)
-      for (int sl = 0; sl < 4 * nw; sl++) sum += red[sl][k];
-    P.rows[(size_t)k * A.rows_cap + b] = sum;
-  }
-}
-
-// ---------------------------------------------------------------------------
 // sums
 // ---------------------------------------------------------------------------
 // Block (k, j): out[j*out_stride + k] = sum over rows r < nrows of column k
@@ -1492,9 +430,6 @@ static int red_grid(int n) {
 // ---------------------------------------------------------------------------
 bool bf_lane_ok(int m, int variant) { return m <= 16 && variant >= 0; }
 
-static int lane_M(int m);
-static size_t mixed_copy_shm(int m, int threads);
-
 // Scratch of matern_tab_fill, in doubles.
 constexpr int kMatScratch = 2 * kMatPieces * kMatN + kMatN * kMatN;
 
@@ -1554,27 +489,6 @@ int bf_rows(const BfArgs &a, const BfConfig &cfg) {
   return need < most ? need : most;
 }
 
-template <int M, bool BATCH>
-static void launch_lane_m(const BfArgs &a, int variant, const dim3 &grid,
-                          const dim3 &blk, hipStream_t st) {
-  // LDS of the block sums: site_terms(nz) doubles a lane
-  const size_t shm =
-      a.rows ? (size_t)blk.x * site_terms(a.nz) * sizeof(double) : 0;
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_bf_lane<M, 0, BATCH>), grid, blk, shm, st, a); break;
-    case 1: hipLaunchKernelGGL((k_bf_lane<M, 1, BATCH>), grid, blk, shm, st, a); break;
-    case kCovMatern15: hipLaunchKernelGGL((k_bf_lane<M, kCovMatern15, BATCH>), grid, blk, shm, st, a); break;
-    case kCovMatern25: hipLaunchKernelGGL((k_bf_lane<M, kCovMatern25, BATCH>), grid, blk, shm, st, a); break;
-    default: hipLaunchKernelGGL((k_bf_lane<M, 3, BATCH>), grid, blk, shm, st, a); break;
-  }
-}
-
-// Per-lane kernel size for m neighbors.
-static int lane_M(int m) {
-  return m <= 4 ? 4 : m <= 8 ? 8 : m <= 10 ? 10 : m <= 12 ? 12 : m <= 15 ? 15
-                                                                          : 16;
-}
-
 // LDS of k_bf_lane_lds: per wavefront, M + 1 rows of zs doubles per lane.
 static size_t lane_lds_shm(int m, int zs, int threads) {
   return (size_t)(threads / 64) * (lane_M(m) + 1) * (zs / 2) * 64 *
@@ -1592,26 +506,6 @@ static bool lane_lds_applies(const BfArgs &a, int threads) {
          lane_lds_shm(a.m, a.zs, threads) <= 65536;
 }
 
-template <int M, int ZH, bool BATCH>
-static void launch_lane_lds_mh(const BfArgs &a, int variant, const dim3 &grid,
-                               const dim3 &blk, size_t shm, hipStream_t st) {
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_bf_lane_lds<M, 0, ZH, BATCH>), grid, blk, shm, st, a); break;
-    case 1: hipLaunchKernelGGL((k_bf_lane_lds<M, 1, ZH, BATCH>), grid, blk, shm, st, a); break;
-    case kCovMatern15: hipLaunchKernelGGL((k_bf_lane_lds<M, kCovMatern15, ZH, BATCH>), grid, blk, shm, st, a); break;
-    case kCovMatern25: hipLaunchKernelGGL((k_bf_lane_lds<M, kCovMatern25, ZH, BATCH>), grid, blk, shm, st, a); break;
-    default: hipLaunchKernelGGL((k_bf_lane_lds<M, 3, ZH, BATCH>), grid, blk, shm, st, a); break;
-  }
-}
-
-template <int M>
-static void launch_lane_lds_m(const BfArgs &a, int variant, const dim3 &grid,
-                              const dim3 &blk, size_t shm, hipStream_t st) {
-  if (a.ng > 0) launch_lane_lds_mh<M, 2, true>(a, variant, grid, blk, shm, st);
-  else if (a.zs == 2) launch_lane_lds_mh<M, 1, false>(a, variant, grid, blk, shm, st);
-  else launch_lane_lds_mh<M, 2, false>(a, variant, grid, blk, shm, st);
-}
-
 static void launch_lane_lds(const BfArgs &a, int variant, const dim3 &grid,
                             const dim3 &blk, hipStream_t st) {
   const size_t shm = lane_lds_shm(a.m, a.zs, (int)blk.x);
@@ -1620,98 +514,6 @@ static void launch_lane_lds(const BfArgs &a, int variant, const dim3 &grid,
     case 12: launch_lane_lds_m<12>(a, variant, grid, blk, shm, st); break;
     case 15: launch_lane_lds_m<15>(a, variant, grid, blk, shm, st); break;
     default: launch_lane_lds_m<16>(a, variant, grid, blk, shm, st); break;
-  }
-}
-
-// LDS of the mixed kernel's covariance copy: (M(M+1)/2 + M) floats a lane.
-static size_t mixed_copy_shm(int m, int threads) {
-  const int M = lane_M(m);
-  return (size_t)threads * (M * (M + 1) / 2 + M) * sizeof(float);
-}
-
-// LDS of the mixed per-lane kernel without the covariance copy: the
-// neighbor offsets.
-static size_t mixed_offsets_shm(int m, int threads) {
-  return (size_t)threads * 2 * lane_M(m) * sizeof(float);
-}
-
-template <int M, bool COPY>
-static void launch_mixed_mc(const BfArgs &a, int variant, const dim3 &grid,
-                            const dim3 &blk, size_t shm, hipStream_t st) {
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_bf_mixed<M, 0, COPY>), grid, blk, shm, st, a); break;
-    case 1: hipLaunchKernelGGL((k_bf_mixed<M, 1, COPY>), grid, blk, shm, st, a); break;
-    case kCovMatern15: hipLaunchKernelGGL((k_bf_mixed<M, kCovMatern15, COPY>), grid, blk, shm, st, a); break;
-    case kCovMatern25: hipLaunchKernelGGL((k_bf_mixed<M, kCovMatern25, COPY>), grid, blk, shm, st, a); break;
-    default: hipLaunchKernelGGL((k_bf_mixed<M, 3, COPY>), grid, blk, shm, st, a); break;
-  }
-}
-
-// Rows of Z that k_bf_mixed_reg stages in LDS: ZH chunks of 16 bytes a
-// row (zs = 2 ZH, Z 16-byte aligned, m > 8 as for the FP64 staging, and the
-// block's stage within 64 KiB), else 0.
-static int mixed_reg_zh(const BfArgs &a, int threads) {
-  if (!a.Z || a.nz <= 0 || a.m <= 8 || ((uintptr_t)a.Z & 15) != 0) return 0;
-  const int zh = a.zs == 2 ? 1 : a.zs == 4 ? 2 : 0;
-  const size_t stage = (size_t)(threads / 64) *
-                       mixed_reg_wave_chunks(lane_M(a.m), zh, a.nz) *
-                       sizeof(double2);
-  return stage <= 65536 ? zh : 0;
-}
-
-static size_t mixed_reg_shm(const BfArgs &a, int threads) {
-  return (size_t)(threads / 64) *
-         mixed_reg_wave_chunks(lane_M(a.m), mixed_reg_zh(a, threads), a.nz) *
-         sizeof(double2);
-}
-
-template <int M, int ZH>
-static void launch_mixed_reg_mh(const BfArgs &a, int variant, const dim3 &grid,
-                                const dim3 &blk, size_t shm, hipStream_t st) {
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_bf_mixed_reg<M, 0, ZH>), grid, blk, shm, st, a); break;
-    case 1: hipLaunchKernelGGL((k_bf_mixed_reg<M, 1, ZH>), grid, blk, shm, st, a); break;
-    case kCovMatern15: hipLaunchKernelGGL((k_bf_mixed_reg<M, kCovMatern15, ZH>), grid, blk, shm, st, a); break;
-    case kCovMatern25: hipLaunchKernelGGL((k_bf_mixed_reg<M, kCovMatern25, ZH>), grid, blk, shm, st, a); break;
-    default: hipLaunchKernelGGL((k_bf_mixed_reg<M, 3, ZH>), grid, blk, shm, st, a); break;
-  }
-}
-
-template <int M>
-static void launch_mixed_reg(const BfArgs &a, int variant, const dim3 &grid,
-                             const dim3 &blk, hipStream_t st) {
-  const size_t shm = mixed_reg_shm(a, (int)blk.x);
-  switch (mixed_reg_zh(a, (int)blk.x)) {
-    case 1: launch_mixed_reg_mh<M, 1>(a, variant, grid, blk, shm, st); break;
-    case 2: launch_mixed_reg_mh<M, 2>(a, variant, grid, blk, shm, st); break;
-    default: launch_mixed_reg_mh<M, 0>(a, variant, grid, blk, shm, st); break;
-  }
-}
-
-// mode 1: the covariance copy in LDS; 3: in registers (one wave per SIMD,
-// covariate rows staged in LDS where they can be); else re-evaluated
-template <int M>
-static void launch_mixed_m(const BfArgs &a, int variant, int mode,
-                           const dim3 &grid, const dim3 &blk, hipStream_t st) {
-  if (mode == 1)
-    launch_mixed_mc<M, true>(a, variant, grid, blk,
-                             mixed_copy_shm(a.m, (int)blk.x), st);
-  else if (mode == 3)
-    launch_mixed_reg<M>(a, variant, grid, blk, st);
-  else
-    launch_mixed_mc<M, false>(a, variant, grid, blk,
-                              mixed_offsets_shm(a.m, (int)blk.x), st);
-}
-
-static void launch_mixed(const BfArgs &a, int variant, int mode,
-                         const dim3 &grid, const dim3 &blk, hipStream_t st) {
-  switch (lane_M(a.m)) {
-    case 4: launch_mixed_m<4>(a, variant, mode, grid, blk, st); break;
-    case 8: launch_mixed_m<8>(a, variant, mode, grid, blk, st); break;
-    case 10: launch_mixed_m<10>(a, variant, mode, grid, blk, st); break;
-    case 12: launch_mixed_m<12>(a, variant, mode, grid, blk, st); break;
-    case 15: launch_mixed_m<15>(a, variant, mode, grid, blk, st); break;
-    default: launch_mixed_m<16>(a, variant, mode, grid, blk, st); break;
   }
 }
 
@@ -1743,27 +545,6 @@ static void launch_coop(const BfArgs &a, const dim3 &grid, const dim3 &blk,
   }
 }
 
-static int launch_grp(const BfArgs &a, const dim3 &grid, const dim3 &blk,
-                      hipStream_t st) {
-  const int waves = (int)blk.x / 64;
-  const int mm = a.m <= 16 ? 16 : 32;
-  const size_t shm = (size_t)waves * grp_wave_doubles(mm) * sizeof(double);
-  const bool mat = a.c.cov == 2;
-  if (mat) {
-    if (!a.mtab) return -2;
-    hipLaunchKernelGGL(k_matern_pieces, dim3(kMpOct), dim3(kMpThreads), 0, st,
-                       a.c, a.mtab);
-  }
-  if (mm == 16) {
-    if (mat) hipLaunchKernelGGL((k_bf_grp<16, true>), grid, blk, shm, st, a);
-    else hipLaunchKernelGGL((k_bf_grp<16, false>), grid, blk, shm, st, a);
-  } else {
-    if (mat) hipLaunchKernelGGL((k_bf_grp<32, true>), grid, blk, shm, st, a);
-    else hipLaunchKernelGGL((k_bf_grp<32, false>), grid, blk, shm, st, a);
-  }
-  return 0;
-}
-
 int bf_launch(const BfArgs &a0, const BfConfig &cfg, int nprob,
               hipStream_t st) {
   if (a0.n <= 0 || nprob <= 0) return 0;
@@ -1790,7 +571,7 @@ int bf_launch(const BfArgs &a0, const BfConfig &cfg, int nprob,
   } else if (cfg.family == 2) {
     if (batch || a.mixed) return -1;  // single FP64 problems only
     a.coop_blocks = nrows;
-    if (const int rc = launch_grp(a, grid, blk, st)) return rc;
+    if (const int rc = bf_row_launch(a, grid, blk, st)) return rc;
   } else {
     a.coop_blocks = nrows;
     const int waves = cfg.threads / 64;

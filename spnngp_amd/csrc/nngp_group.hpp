@@ -2,9 +2,10 @@
 // (four sites per wave), for the general-nu Matern and m > 16, where one
 // site per lane does not fit in registers.
 //
-// Lane u of a row holds rows u and u + 16 of its site's MM x MM system
-// (MM = 16 or 32), so all 64 lanes carry matrix rows; a wavefront-wide
-// system (one site per wave) leaves half of them idle at m = 32.  Within a
+// Lane u of a row holds row u of its site's MM x MM system and, at MM = 32,
+// row 31 - u, so all 64 lanes carry matrix rows (a wavefront-wide system, one
+// site per wave, leaves half of them idle at m = 32) and the two rows of
+// every lane have 31 entries below the diagonal between them.  Within a
 // row, DPP row_newbcast moves a double from lane l to the other 15 lanes
 // in one full-rate instruction (v_mov_b64_dpp), which serves the row's
 // site and, at once, the other three rows' sites: the factor's broadcast
@@ -61,7 +62,7 @@ __device__ __forceinline__ double row_sum16(double x) {
 }
 
 // The system of one site, two rows a lane (the second unused at MM = 16).
-// ra[l] is row u, rb[l] row u + 16; entries above a row's diagonal are
+// ra[l] is row u, rb[l] row 31 - u; entries above a row's diagonal are
 // scratch.  After grp_factor the diagonal holds 1 / L_kk.
 template <int MM>
 struct GrpRows {
@@ -82,7 +83,7 @@ __device__ __forceinline__ bool grp_factor(GrpRows<MM> &S, int u) {
     constexpr int j = decltype(jc)::value;
     double piv;
     if constexpr (j < 16) piv = row_bcast<j>(S.ra[j]);
-    else piv = row_bcast<j - 16>(S.rb[j]);
+    else piv = row_bcast<31 - j>(S.rb[j]);
     ok = ok && (piv > 0.0);
     const double r = nn_rsqrt(piv > 0.0 ? piv : 1.0);
     double la = 0.0, lb = 0.0;
@@ -91,8 +92,8 @@ __device__ __forceinline__ bool grp_factor(GrpRows<MM> &S, int u) {
       S.ra[j] = u == j ? r : la;      // the diagonal keeps 1 / L_jj
     }
     if constexpr (R == 2) {
-      lb = S.rb[j] * r;               // L_(u+16)j
-      S.rb[j] = u + 16 == j ? r : lb;
+      lb = S.rb[j] * r;               // L_(31-u)j
+      S.rb[j] = u == 31 - j ? r : lb;
     }
     if constexpr (j < 15) {
       static_for<j + 1, 16>([&](auto lc) {
@@ -105,7 +106,7 @@ __device__ __forceinline__ bool grp_factor(GrpRows<MM> &S, int u) {
     if constexpr (R == 2) {
       static_for<(j + 1 > 16 ? j + 1 : 16), 32>([&](auto lc) {
         constexpr int l = decltype(lc)::value;
-        const double L = row_bcast<l - 16>(lb);  // L_lj from lane l - 16
+        const double L = row_bcast<31 - l>(lb);  // L_lj from lane 31 - l
         S.rb[l] = fma(-lb, L, S.rb[l]);
       });
     }
@@ -113,8 +114,8 @@ __device__ __forceinline__ bool grp_factor(GrpRows<MM> &S, int u) {
   return ok;
 }
 
-// y = L^-1 (ca, cb) (the lane's rows u and u + 16 of the right-hand side);
-// returns the lane's (y_u, y_u+16).
+// y = L^-1 (ca, cb) (the lane's rows u and 31 - u of the right-hand side);
+// returns the lane's (y_u, y_31-u).
 template <int MM>
 __device__ __forceinline__ void grp_forward(const GrpRows<MM> &S, int u,
                                             double ca, double cb, double &ya,
@@ -131,8 +132,8 @@ __device__ __forceinline__ void grp_forward(const GrpRows<MM> &S, int u,
       aa = fma(-S.ra[k], yk, aa);
       if constexpr (R == 2) ab = fma(-S.rb[k], yk, ab);
     } else {
-      const double yk = row_bcast<k - 16>(ab * S.rb[k]);
-      yb = u + 16 == k ? yk : yb;
+      const double yk = row_bcast<31 - k>(ab * S.rb[k]);
+      yb = u == 31 - k ? yk : yb;
       ab = fma(-S.rb[k], yk, ab);
     }
   });
@@ -140,7 +141,7 @@ __device__ __forceinline__ void grp_forward(const GrpRows<MM> &S, int u,
 
 // B = L^-T y: going down from the last row, the dot product of column k
 // below the diagonal with the B already final is a row sum.  Returns the
-// lane's (B_u, B_u+16).
+// lane's (B_u, B_31-u).
 template <int MM>
 __device__ __forceinline__ void grp_backward(const GrpRows<MM> &S, int u,
                                              double ya, double yb, double &ba,
@@ -152,10 +153,10 @@ __device__ __forceinline__ void grp_backward(const GrpRows<MM> &S, int u,
     constexpr int k = MM - 1 - decltype(qc)::value;
     double s = 0.0;
     if constexpr (k < 16) s = u > k ? S.ra[k] * ba : 0.0;
-    if constexpr (R == 2) s += u + 16 > k ? S.rb[k] * bb : 0.0;
+    if constexpr (R == 2) s += 31 - u > k ? S.rb[k] * bb : 0.0;
     s = row_sum16(s);
     if constexpr (k < 16) ba = u == k ? (ya - s) * S.ra[k] : ba;
-    else bb = u + 16 == k ? (yb - s) * S.rb[k] : bb;
+    else bb = u == 31 - k ? (yb - s) * S.rb[k] : bb;
   });
 }
 
