@@ -418,10 +418,9 @@ typedef struct nngp_tune_report {
                                      refinement residual, 3 = kept in
                                      registers (one wave per SIMD), 0 =
                                      re-evaluated; family 0, FP64:
-                                     2 = the covariate rows of each site's
-                                     neighbors staged in LDS during the
-                                     factorization (same results bit for
-                                     bit as 0)                            */
+                                     2 = finished rows of the factor kept
+                                     in LDS, two waves per SIMD (same
+                                     results bit for bit as 0)            */
   double ms[NNGP_TUNE_MAX];       /* mean launch time                     */
   int best_family, best_threads, best_mode;
 } nngp_tune_report;
@@ -431,7 +430,7 @@ typedef struct nngp_tune_report {
  * and use the fastest for every later pass.  Opt-in: the shape fixes the
  * order of the per-block sums, so a chain is bit-reproducible for a fixed
  * shape; without this call the shape is fixed: the per-lane kernel in
- * 64-thread blocks with the covariate rows staged where it applies, else
+ * 64-thread blocks with finished rows in LDS where it applies, else
  * for FP64 passes with m <= 32 the 16-lane-row kernel in 256-thread blocks,
  * else the wavefront kernel in its widest LDS tile. */
 int nngp_model_autotune(nngp_model *model, const double *theta,

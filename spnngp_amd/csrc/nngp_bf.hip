@@ -455,9 +455,9 @@ bool bf_config_ok(const BfConfig &cfg, int m, int variant) {
          waves <= kCoopMaxWaves && coop_shm(m, waves) <= 65536;
 }
 
-// Untuned passes: per lane at 64 threads with the covariate rows staged
-// in LDS where that applies (the fastest per-lane shape at n = 1e6, m = 15:
-// 0.21 ms a pass against 0.35 ms at 256 threads without staging); else,
+// Untuned passes: per lane at 64 threads with finished rows of the factor
+// in LDS where that applies (the fastest per-lane shape at n = 1e6, m = 15);
+// else,
 // for single FP64 problems with m <= 32, the row kernel at 256 threads
 // (n = 4e6, m = 32, Bessel-K matern: 14.8 ms against 41 ms on the
 // wavefront kernel); else the wavefront kernel.
@@ -489,31 +489,23 @@ int bf_rows(const BfArgs &a, const BfConfig &cfg) {
   return need < most ? need : most;
 }
 
-// LDS of k_bf_lane_lds: per wavefront, M + 1 rows of zs doubles per lane.
-static size_t lane_lds_shm(int m, int zs, int threads) {
-  return (size_t)(threads / 64) * (lane_M(m) + 1) * (zs / 2) * 64 *
-         sizeof(double2);
-}
-
-// Whether an FP64 pass can stage its covariate rows in LDS (mode 2: m > 8,
-// where the factorization is long enough to cover the loads; batched
-// passes with zs = 4 only); where it cannot, mode 2 runs the plain
-// per-lane kernel, whose results are the same bit for bit.
+// Whether an FP64 per-lane pass takes mode 2 (m > 8, where the system is
+// large enough to matter, and the block's LDS within 64 KiB: 64 and 128
+// threads from m = 13 on); where it does not, mode 2 runs the plain per-lane
+// kernel, whose results are the same bit for bit.
 static bool lane_lds_applies(const BfArgs &a, int threads) {
-  return !a.mixed && a.Z && a.nz > 0 && a.m > 8 &&
-         (a.zs == 4 || (a.zs == 2 && a.ng == 0)) &&
-         ((uintptr_t)a.Z & 15) == 0 && (a.ng == 0 || a.fs_Z % 2 == 0) &&
-         lane_lds_shm(a.m, a.zs, threads) <= 65536;
+  return !a.mixed && a.m > 8 &&
+         lane_lds_shm(lane_M(a.m), a.nz, threads) <= 65536;
 }
 
+template <bool BATCH>
 static void launch_lane_lds(const BfArgs &a, int variant, const dim3 &grid,
                             const dim3 &blk, hipStream_t st) {
-  const size_t shm = lane_lds_shm(a.m, a.zs, (int)blk.x);
   switch (lane_M(a.m)) {
-    case 10: launch_lane_lds_m<10>(a, variant, grid, blk, shm, st); break;
-    case 12: launch_lane_lds_m<12>(a, variant, grid, blk, shm, st); break;
-    case 15: launch_lane_lds_m<15>(a, variant, grid, blk, shm, st); break;
-    default: launch_lane_lds_m<16>(a, variant, grid, blk, shm, st); break;
+    case 10: launch_lane_lds_m<10, BATCH>(a, variant, grid, blk, st); break;
+    case 12: launch_lane_lds_m<12, BATCH>(a, variant, grid, blk, st); break;
+    case 15: launch_lane_lds_m<15, BATCH>(a, variant, grid, blk, st); break;
+    default: launch_lane_lds_m<16, BATCH>(a, variant, grid, blk, st); break;
   }
 }
 
@@ -558,15 +550,13 @@ int bf_launch(const BfArgs &a0, const BfConfig &cfg, int nprob,
   const dim3 grid(8 * ((nrows + 7) / 8), nprob);
   const dim3 blk(cfg.threads);
   if (cfg.family == 0) {
+    const bool lds = cfg.mode == 2 && lane_lds_applies(a, cfg.threads);
     if (batch) {
-      if (cfg.mode == 2 && lane_lds_applies(a, cfg.threads))
-        launch_lane_lds(a, variant, grid, blk, st);
-      else
-        launch_lane<true>(a, variant, grid, blk, st);
+      if (lds) launch_lane_lds<true>(a, variant, grid, blk, st);
+      else launch_lane<true>(a, variant, grid, blk, st);
     }
     else if (a.mixed) launch_mixed(a, variant, cfg.mode, grid, blk, st);
-    else if (cfg.mode == 2 && lane_lds_applies(a, cfg.threads))
-      launch_lane_lds(a, variant, grid, blk, st);
+    else if (lds) launch_lane_lds<false>(a, variant, grid, blk, st);
     else launch_lane<false>(a, variant, grid, blk, st);
   } else if (cfg.family == 2) {
     if (batch || a.mixed) return -1;  // single FP64 problems only
@@ -628,7 +618,7 @@ int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
                   // copy (none, LDS, registers); then the wavefront one
     for (int th : {64, 128, 256})
       for (int mode : {0, 1, 3}) cand.push_back(BfConfig{0, th, mode});
-  } else {  // the per-lane kernel: block size x covariate rows in LDS
+  } else {  // the per-lane kernel: block size x factor rows in LDS
     for (int th : {64, 128, 256}) {
       cand.push_back(BfConfig{0, th, 0});
       if (lane_lds_applies(a, th)) cand.push_back(BfConfig{0, th, 2});

@@ -64,6 +64,7 @@ struct BfProblem {
   const double *Z;
   double *rows;
   int *err;
+  int point = 0;  // batched passes: the problem's grid point
 };
 
 template <bool BATCH>
@@ -71,7 +72,9 @@ __device__ __forceinline__ BfProblem bf_problem(const BfArgs &A) {
   BfProblem P{A.xy, A.nnIndx, A.lu, A.Z, A.rows, A.err};
   if constexpr (BATCH) {
     const int j = (int)blockIdx.y;
-    const int f = j / A.ng;
+    // the division's result is known to be uniform only after readfirstlane
+    const int f = __builtin_amdgcn_readfirstlane(j / A.ng);
+    P.point = j - f * A.ng;
     P.xy += (size_t)f * A.fs_xy;
     P.nnIndx += (size_t)f * A.fs_nn;
     P.lu += (size_t)f * A.fs_lu;
@@ -118,6 +121,21 @@ __device__ inline void block_site_terms(int nz, double *rows, int rows_cap,
       for (int ww = 0; ww < nw; ww++) s += red[ww][k];
     rows[(size_t)k * rows_cap + row] = s;
   }
+}
+
+// The parameters at p, the same for every lane of the grid's row, by scalar
+// loads: as an ordinary load they would fill 70 vector registers a lane.  p is
+// not written while the kernel runs.
+__device__ __forceinline__ CovArgs cov_uniform(const CovArgs *p) {
+  static_assert(sizeof(CovArgs) % sizeof(double) == 0, "whole doubles");
+  using Src = const __attribute__((address_space(4))) double *;
+  const Src src = (Src)(uintptr_t)p;
+  CovArgs c;
+  double *d = reinterpret_cast<double *>(&c);
+#pragma unroll
+  for (int k = 0; k < (int)(sizeof(CovArgs) / sizeof(double)); k++)
+    d[k] = src[k];
+  return c;
 }
 
 // Number of per-site terms of a partial row (column 1, always 0, aside):
@@ -209,6 +227,32 @@ inline int lane_M(int m) {
                                                                           : 16;
 }
 
+// Entries of the factor, in packed order, that wait in LDS from the column
+// that finishes their row to the back substitution (row k of L has its last
+// use in the factorization in column k).  Two waves a SIMD leave 256 registers
+// a lane.  Going down the columns, the rows still open, the finished rows, the
+// right-hand side and the coordinates not yet used come to 135 doubles at
+// M = 15 (153 at M = 16); with the first 36 entries in LDS, 99 (117),
+// which fits beside the temporaries, at 18 KB a wave: eight waves take 144
+// of a CU's 160 KB.  Up to M = 12 everything fits in registers.
+// Whole rows: row 7 is the last one kept.
+__host__ __device__ constexpr int lane_lds_entries(int M) {
+  return M <= 12 ? 0 : 36;
+}
+
+// LDS of one wavefront, in doubles: the kept entries or the block sums'
+// terms, whichever is more.
+__host__ __device__ constexpr int lane_wave_doubles(int keep, int nz) {
+  const int sums = site_terms(nz);
+  return 64 * (keep > sums ? keep : (sums + 1) / 2 * 2);
+}
+
+// Dynamic LDS of the per-lane kernel's mode 2, per block.
+inline size_t lane_lds_shm(int M, int nz, int threads) {
+  return (size_t)(threads / 64) * lane_wave_doubles(lane_lds_entries(M), nz) *
+         sizeof(double);
+}
+
 // LDS of the mixed per-lane kernel's covariance copy, per block.
 size_t mixed_copy_shm(int m, int threads);
 
@@ -217,9 +261,9 @@ size_t mixed_copy_shm(int m, int threads);
 template <int M, bool BATCH>
 void launch_lane_m(const BfArgs &a, int variant, const dim3 &grid,
                    const dim3 &blk, hipStream_t st);
-template <int M>
+template <int M, bool BATCH>
 void launch_lane_lds_m(const BfArgs &a, int variant, const dim3 &grid,
-                       const dim3 &blk, size_t shm, hipStream_t st);
+                       const dim3 &blk, hipStream_t st);
 void launch_mixed(const BfArgs &a, int variant, int mode, const dim3 &grid,
                   const dim3 &blk, hipStream_t st);
 

@@ -5,9 +5,11 @@ namespace nngp {
 
 template void launch_lane_m<15, false>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
+template void launch_lane_lds_m<15, false>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 template void launch_lane_m<15, true>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
-template void launch_lane_lds_m<15>(const BfArgs &, int, const dim3 &,
-                                    const dim3 &, size_t, hipStream_t);
+template void launch_lane_lds_m<15, true>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 
 }  // namespace nngp

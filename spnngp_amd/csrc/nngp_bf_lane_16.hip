@@ -5,9 +5,11 @@ namespace nngp {
 
 template void launch_lane_m<16, false>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
+template void launch_lane_lds_m<16, false>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 template void launch_lane_m<16, true>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
-template void launch_lane_lds_m<16>(const BfArgs &, int, const dim3 &,
-                                    const dim3 &, size_t, hipStream_t);
+template void launch_lane_lds_m<16, true>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 
 }  // namespace nngp

@@ -13,9 +13,11 @@ template void launch_lane_m<8, true>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
 template void launch_lane_m<10, false>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
+template void launch_lane_lds_m<10, false>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 template void launch_lane_m<10, true>(const BfArgs &, int, const dim3 &,
                                      const dim3 &, hipStream_t);
-template void launch_lane_lds_m<10>(const BfArgs &, int, const dim3 &,
-                                    const dim3 &, size_t, hipStream_t);
+template void launch_lane_lds_m<10, true>(const BfArgs &, int, const dim3 &,
+                                         const dim3 &, hipStream_t);
 
 }  // namespace nngp

@@ -74,7 +74,7 @@ struct BfConfig {
   int threads = 256;
   int mode = 0;          // mixed-precision passes: 1 = covariance copy in
                          // LDS, 3 = in registers; FP64 per-lane passes:
-                         // 2 = covariate rows staged in LDS
+                         // 2 = finished rows of the factor in LDS
 };
 
 struct BfTuneReport {

@@ -106,8 +106,8 @@ def nn2(coords, coords0, k: int):
 def _shape_name(family, mode):
     """Name of an updateBF launch shape of the autotuner: 'lane' (one site
     per lane; '+lds-copy' and '+reg-copy' for the mixed form's covariance
-    copy in LDS or in registers, '+lds-z' for the FP64 form's covariate rows
-    staged in LDS), 'wave' (one site per wavefront) or 'row' (one site per
+    copy in LDS or in registers, '+lds-z' for the FP64 form that keeps finished
+    rows of the factor in LDS), 'wave' (one site per wavefront) or 'row' (one site per
     16-lane row, four per wavefront)."""
     if family == 0:
         return ("lane", "lane+lds-copy", "lane+lds-z", "lane+reg-copy")[mode]
@@ -498,8 +498,8 @@ class Model:
         (per wavefront) or 2 (per 16-lane row: four sites a wavefront, m <=
         32, FP64), threads per block, and mode as in the autotuner's
         report (1 and 3: the mixed per-lane kernel's covariance copy in LDS
-        or in registers; 2: the FP64 per-lane kernel's covariate rows staged
-        in LDS)."""
+        or in registers; 2: the FP64 per-lane kernel with finished rows of
+        the factor in LDS, at two waves a SIMD)."""
         check(load().nngp_model_set_shape(self._h, int(family), int(threads),
                                           int(mode)))
 
