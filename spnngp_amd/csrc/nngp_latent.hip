@@ -37,6 +37,7 @@
 #include <cstring>
 #include <vector>
 
+#include "nngp_group.hpp"
 #include "nngp_host.hpp"
 
 namespace nngp {
@@ -83,29 +84,28 @@ __global__ __launch_bounds__(kUThreads) void k_u_place(
 // ---------------------------------------------------------------------------
 constexpr int kSweepBlock = 1024;  // the block that walks small phases
 constexpr int kSweepGrid = 256;    // threads per block of a phase's grid
-constexpr int kGridPhase = 4096;   // phases at least this large get a grid
+// Phases at least this large get a grid: a launch costs about 6 us, the time
+// in which one block updates about 500 sites.
+constexpr int kGridPhase = 512;
 
 struct SweepArgs {
   const double *B, *F, *y, *X, *z;
   double *w;
-  const int *nnIndx, *uIndx, *uiIndx, *phase;
-  // per schedule position k: {site i, uIndxLU[i], uIndxLU[n+i], 0}; per
-  // transpose entry t: {nnIndxLU[j], nnIndxLU[n+j]} of the site j = uIndx[t]
-  // (the per-site lookups of the sweep, laid out in the order it reads them)
+  const int *nnIndx, *uIndx, *phase;
+  // per schedule position k: {site i, uIndxLU[i], uIndxLU[n+i], 0} (the
+  // per-site lookups of the sweep, laid out in the order it reads them)
   const int4 *meta;
-  const int2 *uoc;
   // per transpose entry t: B of the site uIndx[t] at its neighbor slot that
   // names the entry's site, gathered from B once per B (k_gather_bt)
   const double *Bt;
   const int *lu;  // nnIndxLU
-  // per site {F_i, r_i}: F of the sweep's B, F slot and the residual
-  // w_i - B_i . w_N(i) at the current w, side by side so that a child's two
-  // values come in one 16 B read
+  // per site {1 / F_i, r_i}: the sweep's F and the residual w_i - B_i .
+  // w_N(i) at the current w, side by side so that a child's two values come
+  // in one 16 B read
   double2 *FR;
+  double *c;  // per site (y_i - x_i . beta) / tau.sq
   double beta[kMaxP];
-  double tau2;
-  unsigned long long seed;  // Philox key when z == nullptr
-  int iter;                 // Philox counter word of this sweep
+  double tau2, itau2;       // tau.sq and 1 / tau.sq
   int n, p, ws;             // w[i * ws]
   int ph0, ph1;             // phases [ph0, ph1)
   int nph;                  // phases in the schedule (phase[] has nph + 1)
@@ -158,91 +158,104 @@ __device__ __forceinline__ double gather_dot(const SweepArgs &A, int o,
 // rounding.)
 //
 // A group of kGroup lanes takes one site; its children are taken kChild at
-// a time, lane l holding children l, l + kGroup, l + 2 kGroup of the chunk,
-// so every load of a chunk is in flight at once.  Every lane adds the
-// children's terms in child order (shuffles) and forms the same draw.  All
-// lanes of a group run the same trip counts.
+// a time, lane l holding children l, l + kGroup, l + 2 kGroup of the chunk.
+// The sums over the children are butterflies of DPP moves, so every lane of
+// the group forms the same draw.  All lanes of a group run the same trip
+// counts.
 constexpr int kGroup = 8;
 constexpr int kPer = 3;
 constexpr int kChild = kGroup * kPer;
 
-__device__ void sweep_site(const SweepArgs &A, int4 mt, int lane) {
-  const int n = A.n, ws = A.ws;
-  double *w = A.w;
-  const int i = mt.x, uo = mt.y, uc = mt.z;
-  const double wi = w[(size_t)i * ws];
-  const double2 fri = A.FR[i];
-  const double fi = fri.x, ri = fri.y;
-  const double yi = A.y[i];
-  double xb = 0.0;
-  for (int q = 0; q < A.p; q++) xb += A.X[(size_t)q * n + i] * A.beta[q];
-  double a = 0.0, v = 0.0;
-  // the first chunk's children (index, B_ji, r_j), kept for the residual
-  // updates; no other site of the phase touches r_j, so the value read here
-  // is still current when it is updated
+// What a site's update needs that no other update of the sweep changes: its
+// first kChild children with their coefficients, its data term, normal and
+// old w.  i < 0: no site.
+struct SweepSite {
+  int i, uo, uc;
   int jk[kPer];
-  double bk[kPer], rk[kPer];
-  for (int j0 = 0; j0 < uc; j0 += kChild) {
-    double ta[kPer], tv[kPer];
+  double bk[kPer];
+  double c, w, z;
+};
+
+// Straight-line code, so that the loads can stay in flight over the previous
+// phase's work; children past the count read the site itself, with a
+// coefficient of 0.
+__device__ __forceinline__ void sweep_fetch(const SweepArgs &A, int4 mt,
+                                            int lane, SweepSite &s) {
+  s.i = mt.x;
+  s.uo = mt.y;
+  s.uc = mt.z;
+  const int ii = mt.x < 0 ? 0 : mt.x;
 #pragma unroll
-    for (int c = 0; c < kPer; c++) {
-      ta[c] = 0.0;
-      tv[c] = 0.0;
-      const int j = j0 + c * kGroup + lane;
-      if (j < uc) {
-        const int t = uo + j;
-        const int jj = A.uIndx[t];
-        const double bij = A.Bt[t];
-        const double2 frj = A.FR[jj];
-        const double fj = frj.x, rj = frj.y;
-        ta[c] = bij * (rj + bij * wi) / fj;
-        tv[c] = bij * bij / fj;
-        if (j0 == 0) {
-          jk[c] = jj;
-          bk[c] = bij;
-          rk[c] = rj;
-        }
-      }
-    }
-    const int nt = min(kChild, uc - j0);
-#pragma unroll
-    for (int t = 0; t < kChild; t++) {
-      if (t < nt) {
-        a += __shfl(ta[t / kGroup], t % kGroup, kGroup);
-        v += __shfl(tv[t / kGroup], t % kGroup, kGroup);
-      }
-    }
+  for (int q = 0; q < kPer; q++) {
+    const int j = q * kGroup + lane;
+    const int t = j < mt.z ? mt.y + j : 0;
+    const int jj = A.uIndx[t];
+    const double b = A.Bt[t];
+    s.jk[q] = j < mt.z ? jj : ii;
+    s.bk[q] = j < mt.z ? b : 0.0;
   }
-  const double e = wi - ri;
-  const double mu = (yi - xb) / A.tau2 + e / fi + a;
-  const double var = 1.0 / (1.0 / A.tau2 + 1.0 / fi + v);
-  const double zi =
-      A.z ? A.z[i] : philox_normal(A.seed, (uint32_t)i, (uint32_t)A.iter);
-  const double wn = mu * var + sqrt(var) * zi;
-  const double d = wn - wi;
+  s.c = A.c[ii];
+  s.w = A.w[(size_t)ii * A.ws];
+  s.z = A.z[ii];
+}
+
+// Sum over the 8 lanes of a group, in every lane.
+__device__ __forceinline__ double group_sum(double x) {
+  static_assert(kGroup == 8, "quad_perm [1,0,3,2], [2,3,0,1], half mirror");
+  x += row_dpp<0xB1>(x);
+  x += row_dpp<0x4E>(x);
+  x += row_dpp<0x141>(x);
+  return x;
+}
+
+// The state that the phases before this one have left for the site's update.
+struct SweepState {
+  double2 fr, frj[kPer];
+};
+
+__device__ __forceinline__ void sweep_state(const SweepArgs &A,
+                                            const SweepSite &s,
+                                            SweepState &t) {
+  t.fr = A.FR[s.i < 0 ? 0 : s.i];
+#pragma unroll
+  for (int q = 0; q < kPer; q++) t.frj[q] = A.FR[s.jk[q]];
+}
+
+__device__ __forceinline__ void sweep_update(const SweepArgs &A,
+                                             const SweepSite &s,
+                                             const SweepState &t, int lane) {
+  if (s.i < 0) return;
+  double a = 0.0, v = 0.0;
+#pragma unroll
+  for (int q = 0; q < kPer; q++) {
+    const double bf = s.bk[q] * t.frj[q].x;
+    a = fma(bf, fma(s.bk[q], s.w, t.frj[q].y), a);
+    v = fma(bf, s.bk[q], v);
+  }
+  for (int j = kChild + lane; j < s.uc; j += kGroup) {
+    const double b = A.Bt[s.uo + j];
+    const double2 fr = A.FR[A.uIndx[s.uo + j]];
+    const double bf = b * fr.x;
+    a = fma(bf, fma(b, s.w, fr.y), a);
+    v = fma(bf, b, v);
+  }
+  a = group_sum(a);
+  v = group_sum(v);
+  const double mu = fma(s.w - t.fr.y, t.fr.x, s.c) + a;
+  const double var = nn_rcp(A.itau2 + t.fr.x + v);
+  const double wn = fma(mu, var, sqrt(var) * s.z);
+  const double d = wn - s.w;
   if (lane == 0) {
-    w[(size_t)i * ws] = wn;
-    A.FR[i].y = ri + d;
+    A.w[(size_t)s.i * A.ws] = wn;
+    A.FR[s.i].y = t.fr.y + d;
   }
-  for (int j0 = 0; j0 < uc; j0 += kChild) {
 #pragma unroll
-    for (int c = 0; c < kPer; c++) {
-      const int j = j0 + c * kGroup + lane;
-      if (j >= uc) continue;
-      int jj;
-      double bij, rj;
-      if (j0 == 0) {
-        jj = jk[c];
-        bij = bk[c];
-        rj = rk[c];
-      } else {
-        const int t = uo + j;
-        jj = A.uIndx[t];
-        bij = A.Bt[t];
-        rj = A.FR[jj].y;
-      }
-      A.FR[jj].y = rj - bij * d;
-    }
+  for (int q = 0; q < kPer; q++)
+    if (q * kGroup + lane < s.uc)
+      A.FR[s.jk[q]].y = fma(-s.bk[q], d, t.frj[q].y);
+  for (int j = kChild + lane; j < s.uc; j += kGroup) {
+    double2 &fr = A.FR[A.uIndx[s.uo + j]];
+    fr.y = fma(-A.Bt[s.uo + j], d, fr.y);
   }
 }
 
@@ -268,33 +281,62 @@ __global__ __launch_bounds__(kSweepGrid) void k_philox_fill(
   if (i < n) z[i] = philox_normal(seed, (uint32_t)i, (uint32_t)iter);
 }
 
-// {F_i, r_i = w_i - B_i . w_N(i)} for every site, before a sweep
+// {1 / F_i, r_i = w_i - B_i . w_N(i)} and the data term of every site, before
+// a sweep
 __global__ __launch_bounds__(kSweepGrid) void k_resid_init(SweepArgs A) {
   const int i = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   if (i >= A.n) return;
-  A.FR[i] = make_double2(A.F[i] * A.fscale,
+  A.FR[i] = make_double2(1.0 / (A.F[i] * A.fscale),
                          A.w[(size_t)i * A.ws] -
                              gather_dot(A, A.lu[i], A.lu[A.n + i], -1));
+  double xb = 0.0;
+  for (int q = 0; q < A.p; q++) xb += A.X[(size_t)q * A.n + i] * A.beta[q];
+  A.c[i] = (A.y[i] - xb) / A.tau2;
 }
 
-// One block walks phases [ph0, ph1) with a barrier between them.  The
-// boundaries of the phase after next and the first site of the next phase
-// are read one phase ahead, so a phase starts with its sites known.
+// One block walks phases [ph0, ph1) with a barrier between them.  The walk is
+// a chain of phases whose length is what bounds it (about 3.2e3 levels of 16
+// sites in site order at n = 5e4), so a phase holds only what depends on the
+// one before: the gather of {1 / F, r}, the group's sums, the draw and the
+// stores.  A phase's sites are read two phases ahead and their children,
+// coefficients and data one phase ahead, with nothing waiting for them, and
+// the sums are DPP butterflies and products with 1 / F.  With those loads,
+// serial shuffled sums and divisions in the phase it took 4.0 us at n = 5e4
+// (12.7 ms a sweep); now 1.0 us.
 __global__ __launch_bounds__(kSweepBlock) void k_sweep_block(SweepArgs A) {
   const int g = (int)threadIdx.x / kGroup, lane = (int)threadIdx.x % kGroup;
   const int ng = (int)blockDim.x / kGroup;
-  int a = A.phase[A.ph0], b = A.phase[A.ph0 + 1];
-  int4 first = a + g < b ? A.meta[a + g] : make_int4(0, 0, 0, 0);
+  const int4 none = make_int4(-1, 0, 0, 0);
+  // boundaries of the phase at hand and the next two: [b0, b1), [b1, b2) ..
+  auto bound = [&](int L) { return A.phase[L < A.nph ? L : A.nph]; };
+  int b0 = bound(A.ph0), b1 = bound(A.ph0 + 1), b2 = bound(A.ph0 + 2),
+      b3 = bound(A.ph0 + 3);
+  SweepSite cur;
+  sweep_fetch(A, b0 + g < b1 ? A.meta[b0 + g] : none, lane, cur);
+  int4 m1 = b1 + g < b2 ? A.meta[b1 + g] : none;
   for (int L = A.ph0; L < A.ph1; L++) {
-    const int c = L + 2 <= A.nph ? A.phase[L + 2] : b;
-    const int4 cur = first;
-    if (b + g < A.n) first = A.meta[b + g];  // checked against c at use
-    for (int k = a + g; k < b; k += ng)
-      sweep_site(A, k == a + g ? cur : A.meta[k], lane);
+    SweepState t;
+    sweep_state(A, cur, t);
+    SweepSite nxt;
+    sweep_fetch(A, m1, lane, nxt);
+    const int mk = b2 + g < b3 ? b2 + g : 0;
+    int4 m2 = A.meta[mk];
+    if (b2 + g >= b3) m2 = none;
+    const int b4 = bound(L + 4);
+    sweep_update(A, cur, t, lane);
+    for (int k = b0 + g + ng; k < b1; k += ng) {  // more sites than groups
+      SweepSite s;
+      sweep_fetch(A, A.meta[k], lane, s);
+      sweep_state(A, s, t);
+      sweep_update(A, s, t, lane);
+    }
     __syncthreads();
-    a = b;
-    b = c;
-    if (a + g >= b) first = make_int4(0, 0, 0, 0);
+    cur = nxt;
+    m1 = m2;
+    b0 = b1;
+    b1 = b2;
+    b2 = b3;
+    b3 = b4;
   }
 }
 
@@ -302,7 +344,12 @@ __global__ __launch_bounds__(kSweepGrid) void k_sweep_grid(SweepArgs A) {
   const int a = A.phase[A.ph0], b = A.phase[A.ph0 + 1];
   const int t = (int)(blockIdx.x * blockDim.x + threadIdx.x);
   const int k = a + t / kGroup;
-  if (k < b) sweep_site(A, A.meta[k], t % kGroup);
+  if (k >= b) return;
+  SweepSite s;
+  SweepState st;
+  sweep_fetch(A, A.meta[k], t % kGroup, s);
+  sweep_state(A, s, st);
+  sweep_update(A, s, st, t % kGroup);
 }
 
 // ---------------------------------------------------------------------------
@@ -315,7 +362,7 @@ constexpr int kLatStats = kMaxP + 1;
 
 struct LatSumArgs {
   const double *y, *X, *w;
-  const double2 *FR;  // {F_i, w_i - B_i . w_N(i)}, current after a sweep
+  const double2 *FR;  // {1 / F_i, w_i - B_i . w_N(i)}, current after a sweep
   double beta[kMaxP];
   double tau2;
   int n, p, ws, mode;  // mode 0: X^T (y - w) / tau.sq and the w quadratic
@@ -347,7 +394,7 @@ __global__ __launch_bounds__(kRedBlock) void k_lat_partial(LatSumArgs A) {
       const double r = (A.y[i] - wi) / A.tau2;
       for (int k = 0; k < A.p; k++) acc[k] += A.X[(size_t)k * n + i] * r;
       const double2 fr = A.FR[i];
-      acc[kMaxP] += fr.y * fr.y / fr.x;
+      acc[kMaxP] += fr.y * fr.y * fr.x;
     } else {
       double xb = 0.0;
       for (int k = 0; k < A.p; k++) xb += A.X[(size_t)k * n + i] * A.beta[k];
@@ -778,13 +825,12 @@ extern "C" int nngp_sNNGP(
                        covModel, opts));
   }
   hipStream_t st = md.st.s;
-  DevBuf dy, dX, du, dui, duoc, dmeta, dR, dphase, dz, dpart, dsum, dwout,
-      dbpos, dBt;
+  DevBuf dy, dX, du, dmeta, dR, dc, dphase, dz, dpart, dsum, dwout, dbpos,
+      dBt;
   NNGP_TRY(dy.alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(dX.alloc(sizeof(double) * (size_t)n * p));
   NNGP_TRY(du.alloc(sizeof(int) * (size_t)std::max(nIndx, 1LL)));
-  NNGP_TRY(dui.alloc(sizeof(int) * (size_t)std::max(nIndx, 1LL)));
-  NNGP_TRY(duoc.alloc(sizeof(int2) * (size_t)std::max(nIndx, 1LL)));
+  NNGP_TRY(dc.alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(dmeta.alloc(sizeof(int4) * (size_t)n));
   NNGP_TRY(dR.alloc(sizeof(double2) * (size_t)n));
   NNGP_TRY(dphase.alloc(sizeof(int) * phase.size()));
@@ -797,18 +843,13 @@ extern "C" int nngp_sNNGP(
   long long ut = 0;
   for (int i = 0; i < n; i++)
     ut = std::max(ut, (long long)uIndxLU[i] + uIndxLU[(size_t)n + i]);
-  std::vector<int2> huoc((size_t)std::max(ut, 1LL));
+  // position in B of each transpose entry's coefficient (entries outside
+  // every site's range are never read; keep them valid)
+  std::vector<int> hbpos((size_t)std::max(ut, 1LL), 0);
   for (long long t = 0; t < ut; t++) {
     const int jj = uIndx[t];
-    // entries outside every site's range are never read; keep them valid
-    const bool ok = jj >= 0 && jj < n;
-    huoc[(size_t)t] = make_int2(ok ? nnIndxLU[jj] : 0,
-                                ok ? nnIndxLU[(size_t)n + jj] : 0);
+    if (jj >= 0 && jj < n) hbpos[(size_t)t] = nnIndxLU[jj] + uiIndx[t];
   }
-  // position in B of each transpose entry's coefficient
-  std::vector<int> hbpos((size_t)std::max(ut, 1LL), 0);
-  for (long long t = 0; t < ut; t++)
-    hbpos[(size_t)t] = huoc[(size_t)t].x + uiIndx[t];
   NNGP_TRY(dbpos.alloc(sizeof(int) * hbpos.size()));
   NNGP_TRY(dBt.alloc(sizeof(double) * hbpos.size()));
   NNGP_HIP(hipMemcpyAsync(dbpos.p, hbpos.data(), dbpos.bytes,
@@ -820,10 +861,6 @@ extern "C" int nngp_sNNGP(
   }
   if (ut > 0) {
     NNGP_HIP(hipMemcpyAsync(du.p, uIndx, sizeof(int) * (size_t)ut,
-                            hipMemcpyHostToDevice, st));
-    NNGP_HIP(hipMemcpyAsync(dui.p, uiIndx, sizeof(int) * (size_t)ut,
-                            hipMemcpyHostToDevice, st));
-    NNGP_HIP(hipMemcpyAsync(duoc.p, huoc.data(), sizeof(int2) * (size_t)ut,
                             hipMemcpyHostToDevice, st));
   }
   NNGP_HIP(hipMemcpyAsync(dmeta.p, hmeta.data(), dmeta.bytes,
@@ -865,16 +902,23 @@ extern "C" int nngp_sNNGP(
   struct Seg {
     int ph0, ph1;
     bool grid;
+    int threads;  // of the block that walks the phases
   };
   std::vector<Seg> segs;
   for (int L = 0; L < nph;) {
     if (phase[(size_t)L + 1] - phase[L] >= kGridPhase) {
-      segs.push_back({L, L + 1, true});
+      segs.push_back({L, L + 1, true, kSweepGrid});
       L++;
     } else {
-      int e = L;
-      while (e < nph && phase[(size_t)e + 1] - phase[e] < kGridPhase) e++;
-      segs.push_back({L, e, false});
+      int e = L, most = 1;
+      while (e < nph && phase[(size_t)e + 1] - phase[e] < kGridPhase) {
+        most = std::max(most, phase[(size_t)e + 1] - phase[e]);
+        e++;
+      }
+      // a group for each site of the largest phase, in whole waves: fewer
+      // waves make the barrier cheaper
+      segs.push_back({L, e, false,
+                      std::min(kSweepBlock, (most * kGroup + 63) / 64 * 64)});
       L = e;
     }
   }
@@ -958,17 +1002,15 @@ extern "C" int nngp_sNNGP(
     A.w = md.Z.as<double>();
     A.nnIndx = md.nnIndx.as<int>();
     A.uIndx = du.as<int>();
-    A.uiIndx = dui.as<int>();
     A.phase = dphase.as<int>();
     A.meta = dmeta.as<int4>();
-    A.uoc = duoc.as<int2>();
     A.Bt = dBt.as<double>();
     A.lu = md.lu.as<int>();
     A.FR = dR.as<double2>();
+    A.c = dc.as<double>();
     for (int k = 0; k < kMaxP; k++) A.beta[k] = k < p ? beta[k] : 0.0;
     A.tau2 = th[1];
-    A.seed = opts ? opts->seed : 1ull;
-    A.iter = s;
+    A.itau2 = 1.0 / th[1];
     A.n = n;
     A.p = p;
     A.ws = md.zs;
@@ -984,8 +1026,8 @@ extern "C" int nngp_sNNGP(
     }
     if (!rng) {
       hipLaunchKernelGGL(k_philox_fill, dim3((n + kSweepGrid - 1) / kSweepGrid),
-                         dim3(kSweepGrid), 0, st, dz.as<double>(), n, A.seed,
-                         A.iter);
+                         dim3(kSweepGrid), 0, st, dz.as<double>(), n,
+                         opts ? opts->seed : 1ull, s);
       NNGP_HIP(hipGetLastError());
     }
     hipLaunchKernelGGL(k_resid_init, dim3((n + kSweepGrid - 1) / kSweepGrid),
@@ -1001,8 +1043,7 @@ extern "C" int nngp_sNNGP(
                            dim3((unsigned)((thr + kSweepGrid - 1) / kSweepGrid)),
                            dim3(kSweepGrid), 0, st, A);
       } else {
-        hipLaunchKernelGGL(k_sweep_block, dim3(1), dim3(kSweepBlock), 0, st,
-                           A);
+        hipLaunchKernelGGL(k_sweep_block, dim3(1), dim3(g.threads), 0, st, A);
       }
       NNGP_HIP(hipGetLastError());
     }
