@@ -54,17 +54,15 @@ static int knn_pred(int n, int m, const double *coords, int *nnIndx,
   NNGP_TRY(use_device(nullptr));
   Stream st;
   NNGP_TRY(st.create());
-  HostStrips h;
-  build_strips(n, coords, coords + n, m, h);
   DevStrips ds;
-  NNGP_TRY(ds.upload(h, st.s));
+  NNGP_TRY(ds.build(coords, n, m, st.s));
   DevBuf xy, dI, dD, dL;
   NNGP_TRY(upload_xy(coords, n, xy, st.s));
   const long long ni = n_indx(n, m);
   NNGP_TRY(dI.alloc(sizeof(int) * (size_t)ni));
   NNGP_TRY(dD.alloc(sizeof(double) * (size_t)ni));
   NNGP_TRY(dL.alloc(sizeof(int) * 2 * (size_t)n));
-  NNGP_TRY(knn_build(coords, n, m, mode, h, ds, xy.as<double2>(), dI.as<int>(),
+  NNGP_TRY(knn_build(coords, n, m, mode, ds, xy.as<double2>(), dI.as<int>(),
                      dD.as<double>(), dL.as<int>(), st.s, nullptr));
   NNGP_HIP(hipMemcpyAsync(nnIndx, dI.p, dI.bytes, hipMemcpyDeviceToHost, st.s));
   NNGP_HIP(hipMemcpyAsync(nnDist, dD.p, dD.bytes, hipMemcpyDeviceToHost, st.s));
@@ -341,10 +339,8 @@ int nngp_nn2(int n, const double *coords, int q, const double *coords0,
   NNGP_TRY(use_device(nullptr));
   Stream st;
   NNGP_TRY(st.create());
-  HostStrips h;
-  build_strips(n, coords, coords + n, k, h);
   DevStrips ds;
-  NNGP_TRY(ds.upload(h, st.s));
+  NNGP_TRY(ds.build(coords, n, k, st.s));
   DevBuf q0, dI, dD;
   NNGP_TRY(upload_xy(coords0, q, q0, st.s));
   NNGP_TRY(dI.alloc(sizeof(int) * (size_t)q * k));

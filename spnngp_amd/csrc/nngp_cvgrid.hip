@@ -547,11 +547,9 @@ int CvGrid::create(const double *yv, const double *X, int p_, int n_,
     NNGP_HIP(hipMemcpyAsync(xy.as<double2>() + (size_t)f * nmod, dxy.p,
                             sizeof(double2) * nmod, hipMemcpyDeviceToDevice,
                             st.s));
-    HostStrips hs;
-    build_strips(nmod, cm.data(), cm.data() + nmod, m, hs);
     DevStrips ds;
-    NNGP_TRY(ds.upload(hs, st.s));
-    NNGP_TRY(knn_build(cm.data(), nmod, m, search, hs, ds, dxy.as<double2>(),
+    NNGP_TRY(ds.build(cm.data(), nmod, m, st.s));
+    NNGP_TRY(knn_build(cm.data(), nmod, m, search, ds, dxy.as<double2>(),
                        nnI.as<int>() + (size_t)f * nn_stride, nullptr,
                        lu.as<int>() + 2 * (size_t)f * nmod, st.s, nullptr));
     // held-out sites and their m nearest training sites

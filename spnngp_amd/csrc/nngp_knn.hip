@@ -337,8 +337,135 @@ int knn_flagged(const unsigned char *flag, int n, int *list, int *count,
   return NNGP_OK;
 }
 
+// ---------------------------------------------------------------------------
+// strip index
+// ---------------------------------------------------------------------------
+__global__ __launch_bounds__(kKnnBlock) void k_iota(int *p, int n) {
+  const int i = blockIdx.x * kKnnBlock + (int)threadIdx.x;
+  if (i < n) p[i] = i;
+}
+
+// The strip of the point at each rank of the x order (ord: nullptr when the
+// points come x-ordered) and the x range of each strip.
+__global__ __launch_bounds__(kKnnBlock) void k_strip_of(
+    const int *ord, const double *x, int n, int S, int *strip_of, double *xlo,
+    double *xhi) {
+  const int r = blockIdx.x * kKnnBlock + (int)threadIdx.x;
+  if (r >= n) return;
+  const int id = ord ? ord[r] : r, t = r / S;
+  strip_of[id] = t;
+  if (r == t * S) xlo[t] = x[id];
+  if (r == t * S + S - 1 || r == n - 1) xhi[t] = x[id];
+}
+
+__global__ __launch_bounds__(kKnnBlock) void k_gather_strip(
+    const int *ids, const int *strip_of, int n, int *out) {
+  const int k = blockIdx.x * kKnnBlock + (int)threadIdx.x;
+  if (k < n) out[k] = strip_of[ids[k]];
+}
+
+__global__ __launch_bounds__(kKnnBlock) void k_gather_xy(
+    const int *ids, const double *x, const double *y, int n, double *sx,
+    double *sy) {
+  const int k = blockIdx.x * kKnnBlock + (int)threadIdx.x;
+  if (k >= n) return;
+  const int id = ids[k];
+  sx[k] = x[id];
+  sy[k] = y[id];
+}
+
+int DevStrips::build(const double *coords, int n, int m, hipStream_t st) {
+  const int S = strip_size(n, m), nstrip = (n + S - 1) / S;
+  sorted = true;
+  for (int i = 1; i < n; i++)
+    if (coords[i] < coords[i - 1]) {
+      sorted = false;
+      break;
+    }
+  // sizes of the sorts' workspaces
+  hipcub::DoubleBuffer<double> kd(nullptr, nullptr);
+  hipcub::DoubleBuffer<int> ki(nullptr, nullptr), vi(nullptr, nullptr);
+  int bits = 1;
+  while (bits < 31 && (1 << bits) < nstrip) bits++;
+  size_t wd = 0, wi = 0;
+  NNGP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, wd, kd, vi, n, 0, 64, st));
+  NNGP_HIP(hipcub::DeviceRadixSort::SortPairs(nullptr, wi, ki, vi, n, 0, bits, st));
+  auto carve = [](size_t &at, size_t bytes) {
+    const size_t o = at;
+    at += (bytes + 255) / 256 * 256;
+    return o;
+  };
+  const size_t nd = sizeof(double) * (size_t)n, ni = sizeof(int) * (size_t)n;
+  size_t keep = 0, work = 0;
+  const size_t o_sx = carve(keep, nd), o_sy = carve(keep, nd),
+               o_id = carve(keep, ni), o_of = carve(keep, ni),
+               o_lo = carve(keep, sizeof(double) * nstrip),
+               o_hi = carve(keep, sizeof(double) * nstrip);
+  const size_t w_xy = carve(work, 2 * nd), w_k0 = carve(work, nd),
+               w_k1 = carve(work, nd), w_v0 = carve(work, ni),
+               w_v1 = carve(work, ni), w_tmp = carve(work, std::max(wd, wi));
+  DevBuf scratch;
+  NNGP_TRY(mem.alloc(keep));
+  NNGP_TRY(scratch.alloc(work));
+  char *kp = mem.as<char>(), *wp = scratch.as<char>();
+  double *x = reinterpret_cast<double *>(wp + w_xy), *y = x + n;
+  double *sx = reinterpret_cast<double *>(kp + o_sx);
+  double *sy = reinterpret_cast<double *>(kp + o_sy);
+  int *sid = reinterpret_cast<int *>(kp + o_id);
+  int *of = reinterpret_cast<int *>(kp + o_of);
+  double *xlo = reinterpret_cast<double *>(kp + o_lo);
+  double *xhi = reinterpret_cast<double *>(kp + o_hi);
+  double *k0 = reinterpret_cast<double *>(wp + w_k0);
+  double *k1 = reinterpret_cast<double *>(wp + w_k1);
+  int *v0 = reinterpret_cast<int *>(wp + w_v0);
+  int *v1 = reinterpret_cast<int *>(wp + w_v1);
+  const dim3 grid((n + kKnnBlock - 1) / kKnnBlock), block(kKnnBlock);
+  NNGP_HIP(hipMemcpyAsync(x, coords, 2 * nd, hipMemcpyHostToDevice, st));
+  // ids by ascending key (one coordinate), ties by id
+  auto by_coordinate = [&](const double *c, const int *&ids) -> int {
+    hipLaunchKernelGGL(k_iota, grid, block, 0, st, v0, n);
+    NNGP_HIP(hipMemcpyAsync(k0, c, nd, hipMemcpyDeviceToDevice, st));
+    hipcub::DoubleBuffer<double> k(k0, k1);
+    hipcub::DoubleBuffer<int> v(v0, v1);
+    size_t b = wd;
+    NNGP_HIP(hipcub::DeviceRadixSort::SortPairs(wp + w_tmp, b, k, v, n, 0, 64, st));
+    ids = v.Current();
+    return NNGP_OK;
+  };
+  const int *ids = nullptr;
+  if (!sorted) NNGP_TRY(by_coordinate(x, ids));
+  hipLaunchKernelGGL(k_strip_of, grid, block, 0, st, ids, (const double *)x, n,
+                     S, of, xlo, xhi);
+  // y order, then stably by strip
+  NNGP_TRY(by_coordinate(y, ids));
+  int *s0 = reinterpret_cast<int *>(k0), *s1 = reinterpret_cast<int *>(k1);
+  hipLaunchKernelGGL(k_gather_strip, grid, block, 0, st, ids, (const int *)of,
+                     n, s0);
+  {
+    int *cur = const_cast<int *>(ids), *alt = cur == v0 ? v1 : v0;
+    hipcub::DoubleBuffer<int> k(s0, s1), v(cur, alt);
+    size_t b = wi;
+    NNGP_HIP(hipcub::DeviceRadixSort::SortPairs(wp + w_tmp, b, k, v, n, 0, bits, st));
+    NNGP_HIP(hipMemcpyAsync(sid, v.Current(), ni, hipMemcpyDeviceToDevice, st));
+  }
+  hipLaunchKernelGGL(k_gather_xy, grid, block, 0, st, (const int *)sid,
+                     (const double *)x, (const double *)y, n, sx, sy);
+  NNGP_HIP(hipGetLastError());
+  NNGP_HIP(hipStreamSynchronize(st));  // the scratch goes away
+  strip_of = of;
+  idx.n = n;
+  idx.S = S;
+  idx.nstrip = nstrip;
+  idx.sx = sx;
+  idx.sy = sy;
+  idx.sid = sid;
+  idx.xlo = xlo;
+  idx.xhi = xhi;
+  return NNGP_OK;
+}
+
 int knn_build(const double *coords, int n, int m, int mode,
-              const HostStrips &h, const DevStrips &ds, const double2 *xy,
+              const DevStrips &ds, const double2 *xy,
               int *nnIndx, double *nnDist, int *lu, hipStream_t st,
               int *nflag_out) {
   DevBuf dFlag, dList, dCount, tmp;
@@ -351,10 +478,10 @@ int knn_build(const double *coords, int n, int m, int mode,
   KnnArgs a;
   a.s = ds.idx;
   a.xy = xy;
-  a.strip_of = ds.strip_of.as<int>();
+  a.strip_of = ds.strip_of;
   a.n = n;
   a.m = m;
-  a.sorted = h.sorted ? 1 : 0;
+  a.sorted = ds.sorted ? 1 : 0;
   a.nnIndx = nnIndx;
   a.nnDist = nnDist;
   a.lu = lu;

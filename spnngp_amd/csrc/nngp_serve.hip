@@ -228,9 +228,7 @@ int Server::create(const double *Xh, const double *yh, const double *coords,
     NNGP_HIP(hipMemcpyAsync(covs.p, hc.data(), covs.bytes, hipMemcpyHostToDevice,
                             s_in.s));
   }
-  HostStrips hs;
-  build_strips(n, coords, coords + n, m, hs);
-  NNGP_TRY(strips.upload(hs, s_in.s));
+  NNGP_TRY(strips.build(coords, n, m, s_in.s));
   NNGP_TRY(arena.alloc(dcap));
   NNGP_TRY(harena.alloc(hcap));
   dalloc.init(dcap);
