@@ -266,8 +266,9 @@ double quad_resid(const PassOut &po, const double *beta, int p);
 // draw() uploads them, walks the neighbor DAG level by level (the level
 // schedule built once by init from the host index) and leaves v in v().
 struct RepDrawer {
-  int n = 0, m = 0, nlev = 0;  // m: the largest neighbor count
-  DevBuf dorder, dloff, dsites, dz, dv, dy;
+  // m: the largest neighbor count, most: sites of the largest level
+  int n = 0, m = 0, nlev = 0, most = 0;
+  DevBuf dorder, dloff, dsites, dz, dv;
   PinnedBuf hz, hv;
   int init(int n, const int *nnIndx, const int *nnIndxLU);
   double *z() { return hz.as<double>(); }

@@ -33,14 +33,32 @@ namespace nngp {
 constexpr int kRepThreads = 1024;
 
 struct RepArgs {
-  const double *B, *F, *z, *X, *beta;
+  const double *B, *e, *X, *beta;  // e: sqrt(F_i) z_i (k_rep_noise)
   const int *nnIndx, *lu, *order, *loff;
   const int4 *sites;  // per position of order: {site, offset, count, 0}
   double *v, *y;
   long long bstride;  // doubles between samples' B
   int n, nlev, p, nS, s0;
-  unsigned long long seed;  // Philox key when z == nullptr
 };
+
+// e[g n + i] = sqrt(F_i) z_i for every site of sample s0 + g (gridDim.y of
+// them), z the caller's normals or, without them, Philox normals keyed by
+// (seed, site, sample).  e may be F itself.  All sites at once: drawn inside
+// the level walk, the ten Philox rounds, the logarithm, the square roots and
+// the cosine sat on the chain of levels (3.1 us a level at n = 1e5, m = 15
+// with them and a 256-thread block; 1.1 us without them and with one wave).
+constexpr int kRepNoise = 256;
+
+__global__ __launch_bounds__(kRepNoise) void k_rep_noise(
+    const double *F, const double *z, int n, int s0, unsigned long long seed,
+    double *e) {
+  const int i = (int)(blockIdx.x * kRepNoise + threadIdx.x);
+  if (i >= n) return;
+  const int g = (int)blockIdx.y;
+  const size_t k = (size_t)g * n + i;
+  e[k] = sqrt(F[k]) *
+         (z ? z[k] : philox_normal(seed, (uint32_t)i, (uint32_t)(s0 + g)));
+}
 
 // Block g: sample s0 + g.  Levels in order; within a level every site's
 // neighbors are final, so its threads may run in any order.
@@ -48,10 +66,8 @@ __global__ __launch_bounds__(kRepThreads) void k_rep_draw(RepArgs A) {
   const int g = (int)blockIdx.x;
   const int n = A.n;
   const double *B = A.B + (size_t)g * A.bstride;
-  const double *F = A.F + (size_t)g * n;
-  const double *z = A.z ? A.z + (size_t)g * n : nullptr;
+  const double *e = A.e + (size_t)g * n;
   double *v = A.v + (size_t)g * n;
-  const int s = A.s0 + g;
   for (int L = 0; L < A.nlev; L++) {
     const int a = A.loff[L], b = A.loff[L + 1];
     for (int k = a + (int)threadIdx.x; k < b; k += (int)blockDim.x) {
@@ -59,29 +75,33 @@ __global__ __launch_bounds__(kRepThreads) void k_rep_draw(RepArgs A) {
       const int off = A.lu[i], cnt = A.lu[n + i];
       double acc = 0.0;
       for (int j = 0; j < cnt; j++) acc += B[off + j] * v[A.nnIndx[off + j]];
-      const double zi =
-          z ? z[i] : philox_normal(A.seed, (uint32_t)i, (uint32_t)s);
-      v[i] = acc + sqrt(F[i]) * zi;
+      v[i] = acc + e[i];
     }
     __syncthreads();
   }
-  // y.rep = v + X beta_s (dgemv at src/rNNGPReplicated.cpp:196)
-  for (int i = (int)threadIdx.x; i < n; i += (int)blockDim.x) {
-    double yi = v[i];
-    for (int j = 0; j < A.p; j++)
-      yi += A.X[(size_t)j * n + i] * A.beta[s + (size_t)j * A.nS];
-    A.y[(size_t)g * n + i] = yi;
-  }
+}
+
+// y.rep = v + X beta_s (dgemv at src/rNNGPReplicated.cpp:196), every site and
+// sample at once (in the walk's one block a sample it cost as much as several
+// hundred levels).
+__global__ __launch_bounds__(kRepNoise) void k_rep_out(RepArgs A) {
+  const int i = (int)(blockIdx.x * kRepNoise + threadIdx.x);
+  if (i >= A.n) return;
+  const int g = (int)blockIdx.y;
+  double yi = A.v[(size_t)g * A.n + i];
+  for (int j = 0; j < A.p; j++)
+    yi += A.X[(size_t)j * A.n + i] * A.beta[A.s0 + g + (size_t)j * A.nS];
+  A.y[(size_t)g * A.n + i] = yi;
 }
 
 // k_rep_draw for m <= M with one site a thread per level.  Slot t of
 // level L is sites[loff[L] + t] = {site, its neighbor offset, count}.  The
-// slot of level L + 2 and the rows of level L + 1 (neighbor ids, B row, F
-// and the normal) are requested while level L waits for its neighbors' v,
+// slot of level L + 2 and the rows of level L + 1 (neighbor ids, B row and
+// noise) are requested while level L waits for its neighbors' v,
 // and nothing waits for them before that wait: each level costs one memory
 // round trip and the barrier.  A level with more sites than threads runs
-// its other sites as k_rep_draw does.  Every site's arithmetic is
-// k_rep_draw's, in the same order.
+// its other sites as k_rep_draw does.  The block is as small as the largest
+// level allows: within one wave the barrier costs nothing.
 constexpr int kRepPfThreads = 256;
 
 template <int M>
@@ -90,7 +110,7 @@ struct RepSlot {
   int cnt;
   int nb[M];
   double b[M];
-  double f, z;  // F_i and the normal
+  double e;  // sqrt(F_i) z_i
 };
 
 __device__ __forceinline__ int4 rep_site(const RepArgs &A, int L, int t) {
@@ -108,8 +128,8 @@ __device__ __forceinline__ int4 rep_site(const RepArgs &A, int L, int t) {
 // 0, 0}) and are then set to 0.
 template <int M>
 __device__ __forceinline__ void rep_rows(const RepArgs &A, const double *B,
-                                         const double *F, const double *z,
-                                         int s, int4 q, RepSlot<M> &r) {
+                                         const double *e, int4 q,
+                                         RepSlot<M> &r) {
   r.i = q.x;
   r.cnt = q.z;
 #pragma unroll
@@ -120,12 +140,7 @@ __device__ __forceinline__ void rep_rows(const RepArgs &A, const double *B,
     r.nb[j] = j < q.z ? nb : 0;
     r.b[j] = j < q.z ? b : 0.0;
   }
-  const int ii = q.x < 0 ? 0 : q.x;
-  const double f = F[ii];
-  const double zz =
-      z ? z[ii] : philox_normal(A.seed, (uint32_t)ii, (uint32_t)s);
-  r.f = q.x < 0 ? 0.0 : f;
-  r.z = q.x < 0 ? 0.0 : zz;
+  r.e = e[q.x < 0 ? 0 : q.x];
 }
 
 template <int M>
@@ -134,13 +149,11 @@ __global__ __launch_bounds__(kRepPfThreads) void k_rep_draw_pf(RepArgs A) {
   const int n = A.n;
   const int t = (int)threadIdx.x;
   const double *B = A.B + (size_t)g * A.bstride;
-  const double *F = A.F + (size_t)g * n;
-  const double *z = A.z ? A.z + (size_t)g * n : nullptr;
+  const double *e = A.e + (size_t)g * n;
   double *v = A.v + (size_t)g * n;
-  const int s = A.s0 + g;
   RepSlot<M> cur, nxt;
   int4 q2 = rep_site(A, 1, t);
-  rep_rows<M>(A, B, F, z, s, rep_site(A, 0, t), cur);
+  rep_rows<M>(A, B, e, rep_site(A, 0, t), cur);
   for (int L = 0; L < A.nlev; L++) {
     // this level's neighbor values first, every slot at once (padded slots
     // read v[0], which no product uses); the loads for the levels ahead go
@@ -149,14 +162,13 @@ __global__ __launch_bounds__(kRepPfThreads) void k_rep_draw_pf(RepArgs A) {
 #pragma unroll
     for (int j = 0; j < M; j++) vn[j] = v[cur.nb[j]];
     const int4 q3 = rep_site(A, L + 2, t);
-    rep_rows<M>(A, B, F, z, s, q2, nxt);
-    // past the count b = 0 and the value is replaced by 0, so those terms
-    // add +0 to a sum that is never -0: the sum is k_rep_draw's bit for bit
-    double acc = 0.0;
+    rep_rows<M>(A, B, e, q2, nxt);
+    // past the count b = 0 and the value is replaced by 0; four partial sums
+    double acc[4] = {cur.e, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int j = 0; j < M; j++)
-      acc += cur.b[j] * (j < cur.cnt ? vn[j] : 0.0);
-    const double vi = acc + sqrt(cur.f) * cur.z;
+      acc[j % 4] = fma(cur.b[j], j < cur.cnt ? vn[j] : 0.0, acc[j % 4]);
+    const double vi = (acc[0] + acc[1]) + (acc[2] + acc[3]);
     if (cur.i >= 0) v[cur.i] = vi;
     const int a = A.loff[L], b = A.loff[L + 1];
     for (int k = a + t + (int)blockDim.x; k < b; k += (int)blockDim.x) {
@@ -164,28 +176,25 @@ __global__ __launch_bounds__(kRepPfThreads) void k_rep_draw_pf(RepArgs A) {
       const int off = A.lu[i], cnt = A.lu[n + i];
       double acc = 0.0;
       for (int j = 0; j < cnt; j++) acc += B[off + j] * v[A.nnIndx[off + j]];
-      const double zi =
-          z ? z[i] : philox_normal(A.seed, (uint32_t)i, (uint32_t)s);
-      v[i] = acc + sqrt(F[i]) * zi;
+      v[i] = acc + e[i];
     }
     __syncthreads();
     cur = nxt;
     q2 = q3;
   }
-  for (int i = t; i < n; i += (int)blockDim.x) {
-    double yi = v[i];
-    for (int j = 0; j < A.p; j++)
-      yi += A.X[(size_t)j * n + i] * A.beta[s + (size_t)j * A.nS];
-    A.y[(size_t)g * n + i] = yi;
-  }
+}
+
+// Threads of the prefetching form for levels of up to `most` sites.
+static int rep_threads(int most) {
+  return most <= 64 ? 64 : most <= 128 ? 128 : kRepPfThreads;
 }
 
 // One block per sample of the group: the prefetching form for m <= 16.
-static void rep_draw_launch(const RepArgs &A, int groups, int m,
+static void rep_draw_launch(const RepArgs &A, int groups, int m, int most,
                             hipStream_t st) {
   if (m <= 16)
-    hipLaunchKernelGGL(k_rep_draw_pf<16>, dim3(groups), dim3(kRepPfThreads),
-                       0, st, A);
+    hipLaunchKernelGGL(k_rep_draw_pf<16>, dim3(groups),
+                       dim3(rep_threads(most)), 0, st, A);
   else
     hipLaunchKernelGGL(k_rep_draw, dim3(groups), dim3(kRepThreads), 0, st,
                        A);
@@ -221,6 +230,14 @@ static int build_levels(int n, const int *nnIndx, const int *lu,
   return NNGP_OK;
 }
 
+// Sites of the largest level.
+static int largest_level(const std::vector<int> &loff) {
+  int most = 0;
+  for (size_t L = 0; L + 1 < loff.size(); L++)
+    most = std::max(most, loff[L + 1] - loff[L]);
+  return most;
+}
+
 // sites[k] = {order[k], its neighbor offset, its count, 0}, on the device.
 static int upload_sites(int n, const int *lu, const std::vector<int> &order,
                         DevBuf &dsites, hipStream_t st) {
@@ -243,6 +260,7 @@ int RepDrawer::init(int n_, const int *nnIndx, const int *lu) {
   std::vector<int> order, loff;
   NNGP_TRY(build_levels(n, nnIndx, lu, order, loff));
   nlev = (int)loff.size() - 1;
+  most = largest_level(loff);
   NNGP_TRY(dorder.alloc(sizeof(int) * (size_t)n));
   NNGP_TRY(dloff.alloc(sizeof(int) * loff.size()));
   NNGP_HIP(hipMemcpy(dorder.p, order.data(), dorder.bytes,
@@ -252,7 +270,6 @@ int RepDrawer::init(int n_, const int *nnIndx, const int *lu) {
   NNGP_TRY(upload_sites(n, lu, order, dsites, nullptr));
   NNGP_TRY(dz.alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(dv.alloc(sizeof(double) * (size_t)n));
-  NNGP_TRY(dy.alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(hz.alloc(sizeof(double) * (size_t)n));
   NNGP_TRY(hv.alloc(sizeof(double) * (size_t)n));
   return NNGP_OK;
@@ -262,29 +279,30 @@ int RepDrawer::draw(const double *B, const double *F, const int *nnIndx,
                     const int *lu, hipStream_t st) {
   NNGP_HIP(hipMemcpyAsync(dz.p, hz.p, sizeof(double) * (size_t)n,
                           hipMemcpyHostToDevice, st));
+  hipLaunchKernelGGL(k_rep_noise, dim3((n + kRepNoise - 1) / kRepNoise),
+                     dim3(kRepNoise), 0, st, F, (const double *)dz.as<double>(),
+                     n, 0, 0ull, dz.as<double>());
   RepArgs A;
   A.B = B;
-  A.F = F;
-  A.z = dz.as<double>();
+  A.e = dz.as<double>();
   A.X = nullptr;
   A.beta = nullptr;
+  A.y = nullptr;  // v itself is the replicate
   A.nnIndx = nnIndx;
   A.lu = lu;
   A.order = dorder.as<int>();
   A.loff = dloff.as<int>();
   A.sites = dsites.as<int4>();
   A.v = dv.as<double>();
-  A.y = dy.as<double>();
   A.bstride = 0;
   A.n = n;
   A.nlev = nlev;
-  A.p = 0;  // y = v
+  A.p = 0;
   A.nS = 1;
   A.s0 = 0;
-  A.seed = 0;
-  rep_draw_launch(A, 1, m, st);
+  rep_draw_launch(A, 1, m, most, st);
   NNGP_HIP(hipGetLastError());
-  NNGP_HIP(hipMemcpyAsync(hv.p, dy.p, sizeof(double) * (size_t)n,
+  NNGP_HIP(hipMemcpyAsync(hv.p, dv.p, sizeof(double) * (size_t)n,
                           hipMemcpyDeviceToHost, st));
   NNGP_HIP(hipStreamSynchronize(st));
   return NNGP_OK;
@@ -315,7 +333,7 @@ extern "C" int nngp_rNNGPReplicated(
   NNGP_TRY(use_device(opts));
   std::vector<int> order, loff;
   NNGP_TRY(build_levels(n, nnIndx, nnIndxLU, order, loff));
-  const int nlev = (int)loff.size() - 1;
+  const int nlev = (int)loff.size() - 1, most = largest_level(loff);
   const int nTheta = covModel == 2 ? 4 : 3;
 
   Model md;  // coordinates and neighbor index resident; no X, y
@@ -461,8 +479,7 @@ extern "C" int nngp_rNNGPReplicated(
     }
     RepArgs A;
     A.B = dB.as<double>();
-    A.F = dF.as<double>();
-    A.z = rng ? dz.as<double>() : nullptr;
+    A.e = dF.as<double>();  // the noise takes F's place
     A.X = dX.as<double>();
     A.beta = dbeta.as<double>();
     A.nnIndx = md.nnIndx.as<int>();
@@ -478,8 +495,13 @@ extern "C" int nngp_rNNGPReplicated(
     A.p = p;
     A.nS = nSamples;
     A.s0 = s0;
-    A.seed = opts ? opts->seed : 1;
-    rep_draw_launch(A, g, m, st);
+    hipLaunchKernelGGL(k_rep_noise, dim3((n + kRepNoise - 1) / kRepNoise, g),
+                       dim3(kRepNoise), 0, st, (const double *)dF.as<double>(),
+                       rng ? (const double *)dz.as<double>() : nullptr, n, s0,
+                       opts ? opts->seed : 1ull, dF.as<double>());
+    rep_draw_launch(A, g, m, most, st);
+    hipLaunchKernelGGL(k_rep_out, dim3((n + kRepNoise - 1) / kRepNoise, g),
+                       dim3(kRepNoise), 0, st, A);
     NNGP_HIP(hipGetLastError());
     if (twobuf) NNGP_TRY(copy_out());  // the previous group, while this one
                                        // computes
