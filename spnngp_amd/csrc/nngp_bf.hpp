@@ -2,6 +2,7 @@
 // problem a block works on, and wavefront sums.
 #pragma once
 #include "nngp_kernels.hpp"
+#include "nngp_lane.hpp"
 #include "nngp_wave.hpp"
 
 namespace nngp {
@@ -123,21 +124,6 @@ __device__ inline void block_site_terms(int nz, double *rows, int rows_cap,
   }
 }
 
-// The parameters at p, the same for every lane of the grid's row, by scalar
-// loads: as an ordinary load they would fill 70 vector registers a lane.  p is
-// not written while the kernel runs.
-__device__ __forceinline__ CovArgs cov_uniform(const CovArgs *p) {
-  static_assert(sizeof(CovArgs) % sizeof(double) == 0, "whole doubles");
-  using Src = const __attribute__((address_space(4))) double *;
-  const Src src = (Src)(uintptr_t)p;
-  CovArgs c;
-  double *d = reinterpret_cast<double *>(&c);
-#pragma unroll
-  for (int k = 0; k < (int)(sizeof(CovArgs) / sizeof(double)); k++)
-    d[k] = src[k];
-  return c;
-}
-
 // Number of per-site terms of a partial row (column 1, always 0, aside):
 // log F, then the nz(nz+1)/2 cross-products.
 __host__ __device__ constexpr int site_terms(int nz) {
@@ -225,19 +211,6 @@ __device__ __forceinline__ void lds_load16(const double *src, double2 *dst) {
 inline int lane_M(int m) {
   return m <= 4 ? 4 : m <= 8 ? 8 : m <= 10 ? 10 : m <= 12 ? 12 : m <= 15 ? 15
                                                                           : 16;
-}
-
-// Entries of the factor, in packed order, that wait in LDS from the column
-// that finishes their row to the back substitution (row k of L has its last
-// use in the factorization in column k).  Two waves a SIMD leave 256 registers
-// a lane.  Going down the columns, the rows still open, the finished rows, the
-// right-hand side and the coordinates not yet used come to 135 doubles at
-// M = 15 (153 at M = 16); with the first 36 entries in LDS, 99 (117),
-// which fits beside the temporaries, at 18 KB a wave: eight waves take 144
-// of a CU's 160 KB.  Up to M = 12 everything fits in registers.
-// Whole rows: row 7 is the last one kept.
-__host__ __device__ constexpr int lane_lds_entries(int M) {
-  return M <= 12 ? 0 : 36;
 }
 
 // LDS of one wavefront, in doubles: the kept entries or the block sums'

@@ -18,14 +18,6 @@ inline int lane_zh(const BfArgs &a) {
 // One site per lane: B_i, F_i and the residual vector e of site i from its
 // neighbor count and offset.  K entries of the factor wait in LDS: pair q of
 // them at keep[q * 64], `keep` the lane's slot in its wavefront's area.
-//
-// The lower triangle is built and factored column by column (left-looking),
-// the covariance entries of a column evaluated when it is reached, so that
-// the M x M system is never held whole: one wave a SIMD, with the whole
-// triangle in registers, left the vector units idle for 30% of the time (the
-// gathers at a wave's start and the chains of dependent instructions).  Each
-// entry goes through the same operations in the same order as in a
-// right-looking factorization, so the results are the same bit for bit.
 // ZH > 0: the rows of Z are ZH aligned pairs (zs = 2 ZH).
 template <int M, int COV, bool BATCH, int ZH, int K>
 __device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
@@ -82,89 +74,39 @@ __device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
     }
   }
 
-  constexpr int T = M * (M + 1) / 2;
-  double a[T];  // packed lower triangle, diagonal as 1 / L_jj
-  double v[M];  // L^-1 c, then B_i
-  double vv = 0.0;
-  bool ok = true;
-#pragma unroll
-  for (int j = 0; j < M; j++) {
-    v[j] = lane_corr<COV>(kBase2 ? lane_d2<COV>(px[j], py[j])
-                                 : sqdist(s.x, s.y, px[j], py[j]),
-                          c);
-#pragma unroll
-    for (int k = j + 1; k < M; k++)
-      a[tri(k, j)] = lane_corr<COV>(
-          lane_d2<COV>(px[k] - px[j], py[k] - py[j]), c);
-    double piv = c.diag;
-#pragma unroll
-    for (int l = 0; l < j; l++) {
-      const double ljl = a[tri(j, l)];
-      piv = fma(-ljl, ljl, piv);
-      v[j] = fma(-ljl, v[l], v[j]);
-#pragma unroll
-      for (int k = j + 1; k < M; k++)
-        a[tri(k, j)] = fma(-a[tri(k, l)], ljl, a[tri(k, j)]);
-    }
-    ok = ok && (piv > 0.0);
-    const double r = nn_rsqrt(piv);
-    a[tri(j, j)] = r;
-#pragma unroll
-    for (int k = j + 1; k < M; k++) a[tri(k, j)] *= r;
-    v[j] *= r;
-    vv = fma(v[j], v[j], vv);
-    // row j is finished: the kept pairs that end in it go to LDS
-#pragma unroll
-    for (int q = 0; q < K / 2; q++)
-      if (2 * q + 1 >= tri(j, 0) && 2 * q + 1 <= tri(j, j))
-        keep[q * 64] = make_double2(a[2 * q], a[2 * q + 1]);
-    // no entry of a later column is evaluated before this column is done
-    __builtin_amdgcn_sched_barrier(0);
-  }
-  Fi = c.diag - vv;
-  // Going back up, the registers of the rows that are done with take what the
-  // residuals need, so that nothing waits for memory after the solve: from
-  // row M - 4 the neighbor slots (again, from cache, rather than held through
-  // the factorization), from row kUp the kept entries and the covariate rows.
-  // The empty asm stands behind the finished rows' work by v[k]; it also
-  // keeps the kept entries from being held in registers since they were
-  // stored, and the loads before it from sinking to their uses.
-  constexpr int kUp = K > 0 ? 7 : M / 2 - 1;
-  static_assert(K == 0 || K == tri(kUp, kUp) + 1, "whole rows are kept");
   const double2 *Z = reinterpret_cast<const double2 *>(P.Z);
   double2 z[ZH > 0 ? ZH : 1], zn[ZH > 0 ? M * ZH : 1];
+  double v[M];  // B_i
+  double vv;
+  const bool ok = lane_solve<M, K, (ZH > 0)>(
+      c.diag,
+      [&](int k, int l) {
+        return lane_corr<COV>(lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);
+      },
+      [&](int k) {
+        return lane_corr<COV>(kBase2 ? lane_d2<COV>(px[k], py[k])
+                                     : sqdist(s.x, s.y, px[k], py[k]),
+                              c);
+      },
+      keep, v, vv,
+      [&] {  // the neighbor slots again (from cache), not held until now
 #pragma unroll
-  for (int k = M - 1; k >= 0; k--) {
-    if (ZH > 0 && k == M - 4) {
-      asm volatile("" : "+v"(v[k]) : : "memory");
+        for (int q = 0; q < M; q++) nb[q] = P.nnIndx[off + q];
+      },
+      [&] {  // the covariate rows
+        if constexpr (ZH > 0) {
 #pragma unroll
-      for (int q = 0; q < M; q++) nb[q] = P.nnIndx[off + q];
-    }
-    if ((K > 0 || ZH > 0) && k == kUp) {
-      asm volatile("" : "+v"(v[k]) : : "memory");
+          for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
 #pragma unroll
-      for (int q = 0; q < K / 2; q++) {
-        const double2 x = keep[q * 64];
-        a[2 * q] = x.x;
-        a[2 * q + 1] = x.y;
-      }
-      if constexpr (ZH > 0) {
+          for (int q = 0; q < M; q++) {
+            const int id = q < cnt ? nb[q] : 0;
 #pragma unroll
-        for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
-#pragma unroll
-        for (int q = 0; q < M; q++) {
-          const int id = q < cnt ? nb[q] : 0;
-#pragma unroll
-          for (int h = 0; h < ZH; h++) zn[q * ZH + h] = Z[(size_t)id * ZH + h];
+            for (int h = 0; h < ZH; h++)
+              zn[q * ZH + h] = Z[(size_t)id * ZH + h];
+          }
         }
-      }
-    }
-    const double t = v[k] * a[tri(k, k)];
-    v[k] = t;
-#pragma unroll
-    for (int l = 0; l < k; l++) v[l] = fma(-a[tri(k, l)], t, v[l]);
-  }
-  if (ZH > 0) asm volatile("" : "+v"(v[0]) : : "memory");
+      });
+  Fi = c.diag - vv;
   if (!BATCH && A.B) {
 #pragma unroll
     for (int k = 0; k < M; k++)

@@ -23,6 +23,7 @@
 #include <cstring>
 
 #include "nngp_host.hpp"
+#include "nngp_lane.hpp"
 #include "nngp_strips.hpp"
 #include "nngp_wave.hpp"
 
@@ -30,7 +31,7 @@ namespace nngp {
 
 constexpr int kSol = 96;        // per-problem solution record (doubles)
 constexpr int kSolA = 8, kSolB = 9, kSolOk = 10, kSolH = 16, kSolV = 32;
-constexpr int kCvPredThreads = 256;
+constexpr int kCvPredThreads = 128;
 constexpr int kCvCoopWaves = 4;
 constexpr int kCvCoopBlocks = 512;
 
@@ -177,9 +178,13 @@ __device__ __forceinline__ double quad_vb(const double *Vb, const double *u,
   return q;
 }
 
+// Waves of the largest block that sums its scores.
+constexpr int kCvMaxWaves =
+    kCvPredThreads / 64 > kCvCoopWaves ? kCvPredThreads / 64 : kCvCoopWaves;
+
 __device__ inline void block_pair_sum(double a, double b, double *prow,
                                       int cap, int row) {
-  __shared__ double red[kCvPredThreads / 64][2];
+  __shared__ double red[kCvMaxWaves][2];
   const int w = (int)threadIdx.x >> 6, t = (int)threadIdx.x & 63;
   const int nw = (int)blockDim.x >> 6;
 #pragma unroll
@@ -199,16 +204,21 @@ __device__ inline void block_pair_sum(double a, double b, double *prow,
   }
 }
 
-// One held-out site per lane (closed-form covariances, m <= 16).
+// One held-out site per lane (closed-form covariances, m <= 16), by the
+// two-wave solve of the updateBF lane kernel (lane_solve): 250 problems of
+// 20,000 sites, m = 15, matern 3/2, took 1.67 ms with the triangle in
+// registers at one wave a SIMD; now 1.04 ms.
 template <int M, int COV>
-__global__ __launch_bounds__(kCvPredThreads) void k_cv_pred_lane(
+__global__ __launch_bounds__(kCvPredThreads, 2) void k_cv_pred_lane(
     CvPredArgs A) {
+  constexpr int K = lane_lds_entries(M);
+  __shared__ double2 area[K > 0 ? kCvPredThreads * K / 2 : 1];
   const int nb = (A.nho + kCvPredThreads - 1) / kCvPredThreads;
   const int b = xcd_block(nb);
   if (b < 0) return;
   const int j = (int)blockIdx.y;
-  const int f = j / A.ng;
-  const CovArgs c = A.covs[j % A.ng];
+  const int f = __builtin_amdgcn_readfirstlane(j / A.ng);
+  const CovArgs c = cov_uniform(A.covs + (j - f * A.ng));
   const double *so = A.sol + (size_t)j * kSol;
   const int i = b * kCvPredThreads + (int)threadIdx.x;
   double crps = 0.0, sq = 0.0;
@@ -222,12 +232,10 @@ __global__ __launch_bounds__(kCvPredThreads) void k_cv_pred_lane(
 #pragma unroll
     for (int k = 0; k < M; k++) {
       if (k < A.m) {
-        nbr[k] = nn0[(size_t)k * A.nho + i];
-        const double2 q = xy[nbr[k]];
+        const double2 q = xy[nn0[(size_t)k * A.nho + i]];
         px[k] = q.x;
         py[k] = q.y;
       } else {  // padding: far away, zero correlation, zero coefficient
-        nbr[k] = 0;
         px[k] = 1e100 * (k + 1);
         py[k] = -1e100 * (k + 1);
       }
@@ -242,21 +250,27 @@ __global__ __launch_bounds__(kCvPredThreads) void k_cv_pred_lane(
         py[k] = (py[k] - s0.y) * c.tsc;
       }
     }
-    constexpr int T = M * (M + 1) / 2;
-    double a[T], v[M];
-#pragma unroll
-    for (int k = 0; k < M; k++) {
-      v[k] = lane_corr<COV>(kBase2 ? lane_d2<COV>(px[k], py[k])
-                                   : sqdist(s0.x, s0.y, px[k], py[k]),
-                            c);
-#pragma unroll
-      for (int l = 0; l < k; l++)
-        a[tri(k, l)] = lane_corr<COV>(
-          lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);
-      a[tri(k, k)] = c.diag;
-    }
+    double v[M];  // w
     double vv;
-    const bool ok = chol_solve<M>(a, v, vv);  // v <- w
+    const bool ok = lane_solve<M, K, true>(
+        c.diag,
+        [&](int k, int l) {
+          return lane_corr<COV>(lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);
+        },
+        [&](int k) {
+          return lane_corr<COV>(kBase2 ? lane_d2<COV>(px[k], py[k])
+                                       : sqdist(s0.x, s0.y, px[k], py[k]),
+                                c);
+        },
+        area + ((int)threadIdx.x >> 6) * (K / 2 * 64) +
+            ((int)threadIdx.x & 63),
+        v, vv,
+        [&] {  // the neighbor slots again (from cache), not held until now
+#pragma unroll
+          for (int k = 0; k < M; k++)
+            nbr[k] = k < A.m ? nn0[(size_t)k * A.nho + i] : 0;
+        },
+        [] {});
     const int p = A.p;
     double u[kMaxP];
     double yhat = 0.0;

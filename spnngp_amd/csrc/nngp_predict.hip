@@ -19,11 +19,13 @@
 //   y0 = x0.beta + w.(y_N - X_N beta),  u = x0 - X_N^T w,
 //   var = b (u^T Vb u + 1 + alpha - w.c0) / (a - 1).
 #include "nngp_kernels.hpp"
+#include "nngp_lane.hpp"
 #include "nngp_wave.hpp"
 
 namespace nngp {
 
-constexpr int kPredBlock = 256;
+constexpr int kPredBlock = 256;   // conjugate predictions
+constexpr int kPredLane = 128;    // samples a block of k_pred_lane
 constexpr int kPredMaxM = 16;
 constexpr int kPredMaxP = kMaxP;
 
@@ -94,11 +96,16 @@ __device__ __forceinline__ double pred_z(const SiteRef &R, int S, int s) {
              : philox_normal(R.seed, (uint32_t)R.i, (uint32_t)s);
 }
 
-// One block = one site x kPredBlock samples.  Grid: (nsite, ceil(S/256)).
+// One block = one site x kPredLane samples.  Grid: (nsite, ceil(S/128)).
 // M >= m; rows m..M-1 are padding at infinite distance (exactly zero
-// correlation), which leaves the real block's arithmetic unchanged.
+// correlation), which leaves the real block's arithmetic unchanged.  The
+// systems are solved at two waves a SIMD (lane_solve): 6,007 sites x 500
+// samples, m = 15, took 760 us with the triangle in registers at one wave;
+// now 578 us.
 template <int M, int COV>
-__global__ __launch_bounds__(kPredBlock) void k_pred_lane(PredArgs A) {
+__global__ __launch_bounds__(kPredLane, 2) void k_pred_lane(PredArgs A) {
+  constexpr int K = lane_lds_entries(M);
+  __shared__ double2 area[K > 0 ? kPredLane * K / 2 : 1];
   __shared__ double sD[M * (M - 1) / 2 + 1];  // pairwise distances (l < k)
   __shared__ double sD0[M];                   // site-neighbor distances
   __shared__ double sY[M];
@@ -132,7 +139,7 @@ __global__ __launch_bounds__(kPredBlock) void k_pred_lane(PredArgs A) {
   if (t < A.p) sX0[t] = R.X0[(size_t)t * R.q + i];
   __syncthreads();
   const double2 s0 = R.xy0[i];
-  for (int p = t; p < M * (M - 1) / 2; p += kPredBlock) {
+  for (int p = t; p < M * (M - 1) / 2; p += kPredLane) {
     int k = 1;
     while ((k + 1) * k / 2 <= p) k++;  // p = k(k-1)/2 + l, l < k
     const int l = p - k * (k - 1) / 2;
@@ -141,7 +148,7 @@ __global__ __launch_bounds__(kPredBlock) void k_pred_lane(PredArgs A) {
   if (t < M) sD0[t] = t < m ? nn_sqrt(sqdist(sPx[t], sPy[t], s0.x, s0.y)) : 1e100;
   __syncthreads();
 
-  const int s = (int)blockIdx.y * kPredBlock + t;
+  const int s = (int)blockIdx.y * kPredLane + t;
   if (s >= A.S) return;
   const double *th = A.theta + (size_t)s * A.nTheta;
   const double s2 = th[0], t2 = th[1], phi = th[2];
@@ -149,19 +156,17 @@ __global__ __launch_bounds__(kPredBlock) void k_pred_lane(PredArgs A) {
   const double phs = phi * A.unit.tsc;  // the unit record's phi is 1
   const bool latent = A.wS != nullptr;
   const double nug = latent ? 0.0 : t2;
-  constexpr int T = M * (M + 1) / 2;
-  double a[T], v[M];
-#pragma unroll
-  for (int k = 0; k < M; k++) {
-    v[k] = s2 * corr_d<COV>(sD0[k], phi, ip, phs, A.unit);
-#pragma unroll
-    for (int l = 0; l < k; l++)
-      a[tri(k, l)] =
-          s2 * corr_d<COV>(sD[k * (k - 1) / 2 + l], phi, ip, phs, A.unit);
-    a[tri(k, k)] = s2 * 1.0 + nug;
-  }
+  double v[M];  // w
   double vv;
-  const bool ok = chol_solve<M>(a, v, vv);  // v <- w
+  const bool ok = lane_solve<M, K, false>(
+      s2 * 1.0 + nug,
+      [&](int k, int l) {
+        return s2 *
+               corr_d<COV>(sD[k * (k - 1) / 2 + l], phi, ip, phs, A.unit);
+      },
+      [&](int k) { return s2 * corr_d<COV>(sD0[k], phi, ip, phs, A.unit); },
+      area + ((int)threadIdx.x >> 6) * (K / 2 * 64) + ((int)threadIdx.x & 63),
+      v, vv, [] {}, [] {});
   const double *bs = A.beta + (size_t)s * A.p;
   double x0b = 0.0;
   for (int j = 0; j < A.p; j++) x0b += sX0[j] * bs[j];
@@ -274,8 +279,8 @@ int pred_launch(const PredArgs &a, hipStream_t st) {
   if (a.nsite <= 0 || a.S <= 0) return 0;
   if (a.p > kPredMaxP) return -1;
   if (a.cov != 2 && a.m <= kPredMaxM) {
-    const dim3 grid(a.nsite, (a.S + kPredBlock - 1) / kPredBlock);
-    const dim3 blk(kPredBlock);
+    const dim3 grid(a.nsite, (a.S + kPredLane - 1) / kPredLane);
+    const dim3 blk(kPredLane);
 #define NNGP_PRED(MM)                                                      \
   do {                                                                    \
     if (a.cov == 0)                                                       \
