@@ -286,14 +286,186 @@ __global__ __launch_bounds__(kKnnBlock) void k_nn2(Nn2Args A) {
   }
 }
 
+// nn2 with one query a wavefront, any k <= 64: lane l holds the l-th smallest
+// (squared distance, row) so far.  A strip is scanned 64 candidates at a time
+// outward from the query's y, and the survivors enter the list one by one (a
+// compare and a lane shift each), so the result is k_nn2's.
+struct WaveList {
+  double d;
+  int id;
+};
+
+__device__ __forceinline__ bool lex_less(double d, int id, double e, int ie) {
+  return d < e || (d == e && id < ie);
+}
+
+__device__ __forceinline__ double lane_value(double x, int lane) {
+  const int lo = __builtin_amdgcn_readlane(__double2loint(x), lane);
+  const int hi = __builtin_amdgcn_readlane(__double2hiint(x), lane);
+  return __hiloint2double(hi, lo);
+}
+
+// Entries of the ascending a[0 .. len) for which below(a[j]) holds (a prefix),
+// 64 probes at a time.
+template <class Below>
+__device__ __forceinline__ int wave_prefix(const double *a, int len, int t,
+                                           Below below) {
+  int lo = 0, hi = len;  // the answer is in [lo, hi]
+  while (lo < hi) {
+    const int step = (hi - lo + 63) / 64;
+    const int j = lo + t * step;
+    const int c = __popcll(__ballot(j < hi && below(a[min(j, len - 1)])));
+    if (c == 0) return lo;
+    const int last = lo + (c - 1) * step;  // below
+    hi = min(hi, last + step);
+    lo = last + 1;
+  }
+  return lo;
+}
+
+__device__ __forceinline__ void wave_scan_strip(const StripIndex &S, int strip,
+                                                double qx, double qy, int self,
+                                                int k, int t, WaveList &L,
+                                                double &worst, int &wid) {
+  const int base = strip * S.S;
+  const int len = min(S.S, S.n - base);
+  const double *sy = S.sy + base;
+  const double *sx = S.sx + base;
+  const int *sid = S.sid + base;
+  // the 64 candidates from j0 on; returns the lanes whose candidate, in range,
+  // has dy^2 within the worst distance
+  auto batch = [&](int j0) {
+    const int j = j0 + t;
+    const bool in = j >= 0 && j < len;
+    const int jc = in ? j : 0;
+    const double dy = qy - sy[jc];
+    const double dx = qx - sx[jc];
+    const int id = sid[jc];
+    const double dy2 = dy * dy, dx2 = dx * dx;
+    const double d2 = dx2 + dy2;
+    unsigned long long left = __ballot(in && (self < 0 || id < self) &&
+                                       lex_less(d2, id, worst, wid));
+    while (left) {
+      const int c = __ffsll((long long)left) - 1;
+      left &= left - 1;
+      const double x = lane_value(d2, c);
+      const int ix = __builtin_amdgcn_readlane(id, c);
+      if (!lex_less(x, ix, worst, wid)) continue;  // the list moved on
+      const bool gt = lex_less(x, ix, L.d, L.id);  // entries behind x
+      const double pd = __shfl_up(L.d, 1);
+      const int pi = __shfl_up(L.id, 1);
+      const bool pgt = t > 0 && lex_less(x, ix, pd, pi);
+      L.d = gt ? (pgt ? pd : x) : L.d;
+      L.id = gt ? (pgt ? pi : ix) : L.id;
+      worst = lane_value(L.d, k - 1);
+      wid = __builtin_amdgcn_readlane(L.id, k - 1);
+    }
+    return __ballot(in && !(dy2 > worst));
+  };
+  const int p = wave_prefix(sy, len, t, [&](double y) { return y < qy; });
+  // the first batch reaches to both sides, so that the worst distance is
+  // small before either side goes on
+  const int a = max(0, min(p - 32, len - 64));
+  const unsigned long long first = batch(a);
+  // each side ends where the farthest of a batch is out of reach (or out of
+  // range, in the side's last batch)
+  unsigned long long up = first, down = first;
+  for (int j = a + 64; j < len && up >> 63; j += 64) up = batch(j);
+  for (int j = a - 64; j > -64 && (down & 1); j -= 64) down = batch(j);
+}
+
+// The k nearest of the query (candidates below `self` only, when self >= 0)
+// outward from strip t0.
+__device__ __forceinline__ WaveList wave_search(const StripIndex &S, int t0,
+                                                double qx, double qy, int self,
+                                                int k, bool left_only, int t) {
+  WaveList L{__builtin_inf(), -1};  // as TopM: unfilled places read -1
+  // The worst distance is wave-uniform and lives in scalar registers; as a
+  // constant, its start would become one s_mov_b64 of a 64-bit literal, which
+  // this compiler emits and the encoding (32 bits) cuts to 0.
+  asm volatile("" : "+v"(L.d), "+v"(L.id));
+  double worst = lane_value(L.d, k - 1);
+  int wid = __builtin_amdgcn_readlane(L.id, k - 1);
+  wave_scan_strip(S, t0, qx, qy, self, k, t, L, worst, wid);
+  for (int s = t0 - 1; s >= 0; s--) {
+    const double gap = qx - S.xhi[s];
+    if (gap > 0.0 && gap * gap > worst) break;
+    wave_scan_strip(S, s, qx, qy, self, k, t, L, worst, wid);
+  }
+  if (left_only) return L;
+  for (int s = t0 + 1; s < S.nstrip; s++) {
+    const double gap = S.xlo[s] - qx;
+    if (gap > 0.0 && gap * gap > worst) break;
+    wave_scan_strip(S, s, qx, qy, self, k, t, L, worst, wid);
+  }
+  return L;
+}
+
+__global__ __launch_bounds__(kKnnBlock) void k_nn2_wave(Nn2Args A) {
+  const int i = __builtin_amdgcn_readfirstlane(
+      (int)((blockIdx.x * kKnnBlock + threadIdx.x) >> 6));
+  const int t = (int)threadIdx.x & 63;
+  if (i >= A.nq) return;
+  const double2 q = A.q[i];
+  // the last strip with xlo <= x, else the first
+  const int t0 = max(0, wave_prefix(A.s.xlo, A.s.nstrip, t,
+                                    [&](double x) { return x <= q.x; }) - 1);
+  const WaveList L = wave_search(A.s, t0, q.x, q.y, -1, A.k, false, t);
+  if (t < A.k) {
+    const size_t o = (size_t)t * A.nq + i;
+    A.idx[o] = L.id;
+    if (A.dist) A.dist[o] = sqrt(L.d);
+  }
+}
+
+// k_knn_pred with one site a wavefront (m + 1 <= 64 candidates, one a lane).
+// n = 1e6, m = 15: 9.6 ms with one lane a site, whose every accepted candidate
+// moves a 16-entry list of all 64 lanes; now 3.4 ms.  n = 5e5 clustered, m =
+// 32: 9.7 and 2.7 ms.
+__global__ __launch_bounds__(kKnnBlock) void k_knn_pred_wave(KnnArgs A) {
+  const int i = __builtin_amdgcn_readfirstlane(
+      (int)((blockIdx.x * kKnnBlock + threadIdx.x) >> 6));
+  const int t = (int)threadIdx.x & 63;
+  if (i >= A.n) return;
+  int off, cnt;
+  nn_layout(i, A.m, off, cnt);
+  if (t == 0) {
+    A.lu[i] = off;
+    A.lu[A.n + i] = cnt;
+    if (cnt == 0) A.flag[i] = 0;
+  }
+  if (cnt == 0) return;
+  const int cs = min(i, A.m + 1);
+  const double2 q = A.xy[i];
+  const WaveList L = wave_search(A.s, A.strip_of[i], q.x, q.y, i, cs,
+                                 A.sorted != 0, t);
+  // k_knn_pred's rule for the replay, on lanes t and t + 1 < cs
+  const double d = A.mode == 0 ? L.d : sqrt(L.d);
+  const double nd = __shfl_down(d, 1);
+  bool tie;
+  if (A.mode == 0) {
+    const double dmax = lane_value(L.d, cs - 1);
+    const double g =
+        ldexp(dmax, -40) + 2.0 * sqrt(2.0 * dmax) * A.E + A.E * A.E;
+    tie = nd - d <= g;
+  } else {
+    tie = nd == d;
+  }
+  const bool flag = __ballot(t + 1 < cs && tie) != 0;
+  if (t == 0) A.flag[i] = flag ? 1 : 0;
+  if (t < cnt) {
+    A.nnIndx[off + t] = L.id;
+    if (A.nnDist) A.nnDist[off + t] = sqrt(L.d);
+  }
+}
+
 int knn_launch(const KnnArgs &a, hipStream_t st) {
-  const dim3 grid((a.n + kKnnBlock - 1) / kKnnBlock), block(kKnnBlock);
-  if (a.m < 16)
-    hipLaunchKernelGGL(k_knn_pred<16>, grid, block, 0, st, a);
-  else if (a.m < 33)
-    hipLaunchKernelGGL(k_knn_pred<33>, grid, block, 0, st, a);
-  else if (a.m < 65)
-    hipLaunchKernelGGL(k_knn_pred<65>, grid, block, 0, st, a);
+  const dim3 block(kKnnBlock);
+  if (a.m < 64)
+    hipLaunchKernelGGL(k_knn_pred_wave, dim3((a.n + 3) / 4), block, 0, st, a);
+  else if (a.m < 65)  // 65 candidates: one site a lane
+    hipLaunchKernelGGL(k_knn_pred<65>, dim3((a.n + kKnnBlock - 1) / kKnnBlock),
+                       block, 0, st, a);
   else
     return -1;
   return (int)hipGetLastError();
@@ -554,17 +726,21 @@ int knn_build(const double *coords, int n, int m, int mode,
   return NNGP_OK;
 }
 
+// Queries up to which nn2 gives each a wavefront when k <= 16: about 4.5 us a
+// thousand queries, against 150 to 280 us for one query a lane whatever their
+// number (n = 2e3 to 1e6, k = 10 and 15).  For k > 16 the lanes' 32- and
+// 64-entry lists took 2 to 6 ms, against 7 us a thousand.
+constexpr int kNn2Wave = 49152;
+
 int nn2_launch(const Nn2Args &a, hipStream_t st) {
   if (a.nq <= 0) return 0;
-  const dim3 grid((a.nq + kKnnBlock - 1) / kKnnBlock), block(kKnnBlock);
-  if (a.k <= 16)
-    hipLaunchKernelGGL(k_nn2<16>, grid, block, 0, st, a);
-  else if (a.k <= 32)
-    hipLaunchKernelGGL(k_nn2<32>, grid, block, 0, st, a);
-  else if (a.k <= 64)
-    hipLaunchKernelGGL(k_nn2<64>, grid, block, 0, st, a);
+  if (a.k > 64) return -1;
+  const dim3 block(kKnnBlock);
+  if (a.k > 16 || a.nq <= kNn2Wave)
+    hipLaunchKernelGGL(k_nn2_wave, dim3((a.nq + 3) / 4), block, 0, st, a);
   else
-    return -1;
+    hipLaunchKernelGGL(k_nn2<16>, dim3((a.nq + kKnnBlock - 1) / kKnnBlock),
+                       block, 0, st, a);
   return (int)hipGetLastError();
 }
 
