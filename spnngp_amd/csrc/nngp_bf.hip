@@ -34,6 +34,7 @@
 // partial row, and k_rows_sum adds the rows of each column in a fixed order.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <climits>
 #include <cstdint>
 #include <map>
@@ -591,8 +592,8 @@ int bf_sums_launch(const BfArgs &a, const BfConfig &cfg, int nprob,
 // Candidates: sites per wavefront (64: the per-lane kernel at 64, 128 or
 // 256 threads per block; 1: the wavefront kernel with 1, 2 or 4 waves per
 // block, i.e. LDS tiles of 1, 2 or 4 systems).  Each is timed with HIP
-// events on the caller's stream (one warm-up, then `reps` launches) and the
-// fastest kept.  Results are cached per (m, variant, nz, size class).
+// events on the caller's stream (one warm-up, then three launches; fewer
+// where it is far behind) and the fastest kept.  Results are cached per (m, variant, nz, size class).
 namespace {
 std::mutex g_tune_mu;
 std::map<std::tuple<int, int, int, int>, BfConfig> g_tune_cache;
@@ -633,23 +634,37 @@ int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
     (void)hipEventDestroy(e0);
     return -1;
   }
-  const int reps = 3;
-  double best_ms = 1e300;
+  // mean time of `reps` launches after one more
+  auto timed = [&](const BfConfig &cfg, int np, int reps, double *per) -> int {
+    int e = bf_launch(a, cfg, np, st);
+    if (!e) e = (int)hipEventRecord(e0, st);
+    for (int r = 0; r < reps && !e; r++) e = bf_launch(a, cfg, np, st);
+    if (!e) e = (int)hipEventRecord(e1, st);
+    if (!e) e = (int)hipEventSynchronize(e1);
+    float ms = 0.0f;
+    if (!e) e = (int)hipEventElapsedTime(&ms, e0, e1);
+    *per = ms / reps;
+    return e;
+  };
+  double best_ms = 1e300, best_few = 1e300;
   BfConfig pick = bf_default(a.m, variant, !a.mixed && a.ng == 0);
   int nc = 0;
   int rc = 0;
   for (const BfConfig &cfg : cand) {
     if (!bf_config_ok(cfg, a.m, variant)) continue;
     if (a.rows && bf_rows(a, cfg) > a.rows_cap) continue;
-    if ((rc = bf_launch(a, cfg, nprob, st)) != 0) break;
-    if ((rc = (int)hipEventRecord(e0, st)) != 0) break;
-    for (int r = 0; r < reps && rc == 0; r++) rc = bf_launch(a, cfg, nprob, st);
+    double per = 0.0;
+    // a candidate that a sixteenth of the problems (or the one problem) shows
+    // to be half as fast as another is not timed further: the wavefront shapes
+    // of a 250-problem grid cost 370 of its first run's 393 ms
+    const int few = std::max(1, nprob / 16);
+    if ((rc = timed(cfg, few, 1, &per)) != 0) break;
+    best_few = std::min(best_few, per);
+    if (per < 2.0 * best_few)
+      rc = timed(cfg, nprob, 3, &per);
+    else
+      per *= (double)nprob / few;
     if (rc) break;
-    if ((rc = (int)hipEventRecord(e1, st)) != 0) break;
-    if ((rc = (int)hipEventSynchronize(e1)) != 0) break;
-    float ms = 0.0f;
-    if ((rc = (int)hipEventElapsedTime(&ms, e0, e1)) != 0) break;
-    const double per = ms / reps;
     if (rep && nc < NNGP_TUNE_MAX) {
       rep->family[nc] = cfg.family;
       rep->threads[nc] = cfg.threads;
