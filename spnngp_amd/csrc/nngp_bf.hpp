@@ -198,15 +198,6 @@ __device__ inline void block_site_terms_lds(int nz, double *rows,
   }
 }
 
-// Direct-to-LDS load of 16 bytes a lane: lane t's bytes land at dst + t
-// (dst the same for the whole wavefront).  The load counts in vmcnt like any
-// other; the data are in LDS once it has been waited for.
-__device__ __forceinline__ void lds_load16(const double *src, double2 *dst) {
-  __builtin_amdgcn_global_load_lds(
-      (const __attribute__((address_space(1))) void *)src,
-      (__attribute__((address_space(3))) void *)dst, 16, 0, 0);
-}
-
 // Per-lane kernel size for m neighbors.
 inline int lane_M(int m) {
   return m <= 4 ? 4 : m <= 8 ? 8 : m <= 10 ? 10 : m <= 12 ? 12 : m <= 15 ? 15

@@ -194,40 +194,38 @@ __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed(BfArgs A) {
   if (A.rows) block_site_terms(A.nz, A.rows, A.rows_cap, valid, Fi, e, b);
 }
 
-// k_bf_mixed's scheme at one wave per SIMD, where the FP32 factor and a
-// register copy of C both fit: no entry is evaluated twice and C does not
-// go through LDS.  The arithmetic is k_bf_mixed's step for step, so B and F
-// equal its results bit for bit.  As in lane_site, ZH > 0 stages the
-// covariate rows of the M neighbor slots and of the site in LDS with the
-// coordinate gathers (chunk h of slot k at stg[(k * ZH + h) * 64 + lane]).
+// k_bf_mixed's scheme with a copy of C kept, so that no entry is evaluated
+// twice: what of the copy the registers of two waves per SIMD cannot hold
+// beside the factor waits in LDS for the residual (mixed_lds_entries, four
+// entries a lane in each 16 bytes).  The arithmetic is k_bf_mixed's step for
+// step, so B and F equal its results bit for bit.  With the whole copy in
+// registers, one wave per SIMD and the covariate rows staged in LDS, a pass
+// took 155 us at n = 1e6, m = 15 (the vector units busy 61% of the time);
+// now 120 us.  ZH > 0: the rows of Z are ZH aligned pairs.
+__host__ __device__ constexpr int mixed_lds_entries(int M) {
+  return M <= 12 ? 0 : 72;
+}
+
 template <int M, int COV, int ZH>
 __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
                                                int cnt, int off,
                                                int (&nb)[M], double &Fi,
                                                double (&e)[kMaxNZ],
-                                               double2 *stg) {
+                                               float4 *keep) {
+  constexpr int K = mixed_lds_entries(M);
   const CovArgs &c = A.c;
   const CovArgs32 c32 = cov32(c);
   if (cnt == 0) {  // site 0: F = s2 + t2, residual = the data
     Fi = c.diag;
 #pragma unroll
-    for (int j = 0; j < kMaxNZ; j++)
-      if (j < A.nz) e[j] = A.Z[(size_t)i * A.zs + j];
+    for (int j = 0; j < (ZH > 0 ? 2 * ZH : kMaxNZ); j++)
+      if (ZH > 0 || j < A.nz) e[j] = A.Z[(size_t)i * A.zs + j];
     return;
   }
   if (cnt < M) {
 #pragma unroll
     for (int k = 0; k < M; k++)
       if (k >= cnt) nb[k] = 0;
-  }
-  if constexpr (ZH > 0) {
-#pragma unroll
-    for (int k = 0; k <= M; k++) {
-      const double *zr = A.Z + (size_t)(k < M ? nb[k] : i) * (2 * ZH);
-#pragma unroll
-      for (int h = 0; h < ZH; h++)
-        lds_load16(zr + 2 * h, stg + (k * ZH + h) * 64);
-    }
   }
   const double2 s = A.xy[i];
   float dx[M], dy[M];
@@ -247,20 +245,36 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
     }
   }
   constexpr int T = M * (M + 1) / 2;
-  float a[T], ac[T], v[M], cv[M];
+  float a[T], v[M], cv[M];
+  float ac[M * (M - 1) / 2];  // C below the diagonal, row by row
 #pragma unroll
   for (int k = 0; k < M; k++) {
     v[k] = s2_corr32<COV>(fmaf(dx[k], dx[k], dy[k] * dy[k]), c32);
     cv[k] = v[k];
 #pragma unroll
     for (int l = 0; l < k; l++) {
-      a[tri(k, l)] = pair32<COV>(dx[k], dy[k], dx[l], dy[l], c32);
-      ac[tri(k, l)] = a[tri(k, l)];
+      const int q = k * (k - 1) / 2 + l;
+      ac[q] = pair32<COV>(dx[k], dy[k], dx[l], dy[l], c32);
+      a[tri(k, l)] = ac[q];
+      if (q < K && q % 4 == 3)
+        keep[q / 4 * 64] = make_float4(ac[q - 3], ac[q - 2], ac[q - 1], ac[q]);
     }
     a[tri(k, k)] = c32.diag;
   }
   const bool ok = chol_factor32<M>(a);
   chol_apply32<M>(a, v);  // v <- B0
+  if constexpr (K > 0) {
+    // the kept entries come from LDS, not from registers held until here
+    asm volatile("" : "+v"(v[0]) : : "memory");
+#pragma unroll
+    for (int q = 0; q < K / 4; q++) {
+      const float4 x = keep[q * 64];
+      ac[4 * q] = x.x;
+      ac[4 * q + 1] = x.y;
+      ac[4 * q + 2] = x.z;
+      ac[4 * q + 3] = x.w;
+    }
+  }
   // residual r = c - C B0 in FP64
   double r[M];
   const double dg = (double)c32.diag;
@@ -270,11 +284,15 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
   for (int k = 1; k < M; k++) {
 #pragma unroll
     for (int l = 0; l < k; l++) {
-      const double ckl = (double)ac[tri(k, l)];
+      const double ckl = (double)ac[k * (k - 1) / 2 + l];
       r[k] = fma(-ckl, (double)v[l], r[k]);
       r[l] = fma(-ckl, (double)v[k], r[l]);
     }
   }
+  // the neighbor slots again (from cache), in time for the covariate rows
+  asm volatile("" : "+v"(r[0]) : : "memory");
+#pragma unroll
+  for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
   float d[M];
 #pragma unroll
   for (int k = 0; k < M; k++) d[k] = (float)r[k];
@@ -293,20 +311,26 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
   }
   Fi = c.diag - cb;
   // residual vectors; padded coefficients are 0
+#pragma unroll
+  for (int k = 0; k < M; k++) nb[k] = k < cnt ? nb[k] : 0;
   if constexpr (ZH > 0) {
-    const int t = (int)threadIdx.x & 63;
+    const double2 *Z = reinterpret_cast<const double2 *>(A.Z);
+    double2 z[ZH];
+#pragma unroll
+    for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
+#pragma unroll
+    for (int k = 0; k < M; k++) {
+#pragma unroll
+      for (int h = 0; h < ZH; h++) {
+        const double2 q = Z[(size_t)nb[k] * ZH + h];
+        z[h].x = fma(-bd[k], q.x, z[h].x);
+        z[h].y = fma(-bd[k], q.y, z[h].y);
+      }
+    }
 #pragma unroll
     for (int h = 0; h < ZH; h++) {
-      const double2 zi = stg[(M * ZH + h) * 64 + t];
-      double e0 = zi.x, e1 = zi.y;
-#pragma unroll
-      for (int k = 0; k < M; k++) {
-        const double2 z = stg[(k * ZH + h) * 64 + t];
-        e0 = fma(-bd[k], z.x, e0);
-        e1 = fma(-bd[k], z.y, e1);
-      }
-      e[2 * h] = e0;
-      e[2 * h + 1] = e1;
+      e[2 * h] = z[h].x;
+      e[2 * h + 1] = z[h].y;
     }
   } else {
 #pragma unroll
@@ -323,16 +347,16 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
   if (!ok || !(Fi > 0.0)) atomicMin(A.err, i);
 }
 
-// Dynamic LDS of k_bf_mixed_reg a wavefront, in double2: the staged rows,
-// which the block sums then reuse, or the sums' area alone.
-__host__ __device__ inline int mixed_reg_wave_chunks(int M, int ZH, int nz) {
+// Dynamic LDS of k_bf_mixed_reg a wavefront, in double2: the kept entries,
+// which the block sums then overwrite, or the sums' terms.
+__host__ __device__ inline int mixed_reg_wave_chunks(int M, int nz) {
   const int sums = (site_terms(nz) * 64 + 1) / 2;
-  const int stage = (M + 1) * ZH * 64;
-  return stage > sums ? stage : sums;
+  const int keep = mixed_lds_entries(M) / 4 * 64;
+  return keep > sums ? keep : sums;
 }
 
 template <int M, int COV, int ZH>
-__global__ __launch_bounds__(kLaneMaxThreads) void k_bf_mixed_reg(BfArgs A) {
+__global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed_reg(BfArgs A) {
   extern __shared__ double2 mstage[];
   const int nt = (int)blockDim.x;
   const int b = xcd_block((A.n + nt - 1) / nt);
@@ -340,7 +364,7 @@ __global__ __launch_bounds__(kLaneMaxThreads) void k_bf_mixed_reg(BfArgs A) {
   const int i = b * nt + (int)threadIdx.x;
   const bool valid = i < A.n;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  double2 *stg = mstage + (size_t)w * mixed_reg_wave_chunks(M, ZH, A.nz);
+  double2 *stg = mstage + (size_t)w * mixed_reg_wave_chunks(M, A.nz);
   double Fi = 1.0;
   double e[kMaxNZ];
 #pragma unroll
@@ -356,7 +380,9 @@ __global__ __launch_bounds__(kLaneMaxThreads) void k_bf_mixed_reg(BfArgs A) {
     int nb[M];
 #pragma unroll
     for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
-    mixed_reg_site<M, COV, ZH>(A, i, cnt, off, nb, Fi, e, stg);
+    mixed_reg_site<M, COV, ZH>(
+        A, i, cnt, off, nb, Fi, e,
+        reinterpret_cast<float4 *>(stg) + ((int)threadIdx.x & 63));
     if (A.F) A.F[i] = Fi;
   }
   if (A.rows)
@@ -388,21 +414,16 @@ static void launch_mixed_mc(const BfArgs &a, int variant, const dim3 &grid,
   }
 }
 
-// Rows of Z that k_bf_mixed_reg stages in LDS: ZH chunks of 16 bytes a
-// row (zs = 2 ZH, Z 16-byte aligned, m > 8 as for the FP64 staging, and the
-// block's stage within 64 KiB), else 0.
+// Aligned pairs in a row of Z that k_bf_mixed_reg reads (zs = 2 ZH, Z 16-byte
+// aligned, m > 8), else 0: single values, as also for rows of two pairs in
+// 256-thread blocks, a shape that smaller blocks beat.
 static int mixed_reg_zh(const BfArgs &a, int threads) {
   if (!a.Z || a.nz <= 0 || a.m <= 8 || ((uintptr_t)a.Z & 15) != 0) return 0;
-  const int zh = a.zs == 2 ? 1 : a.zs == 4 ? 2 : 0;
-  const size_t stage = (size_t)(threads / 64) *
-                       mixed_reg_wave_chunks(lane_M(a.m), zh, a.nz) *
-                       sizeof(double2);
-  return stage <= 65536 ? zh : 0;
+  return a.zs == 2 ? 1 : a.zs == 4 && threads <= 128 ? 2 : 0;
 }
 
 static size_t mixed_reg_shm(const BfArgs &a, int threads) {
-  return (size_t)(threads / 64) *
-         mixed_reg_wave_chunks(lane_M(a.m), mixed_reg_zh(a, threads), a.nz) *
+  return (size_t)(threads / 64) * mixed_reg_wave_chunks(lane_M(a.m), a.nz) *
          sizeof(double2);
 }
 
@@ -429,8 +450,8 @@ static void launch_mixed_reg(const BfArgs &a, int variant, const dim3 &grid,
   }
 }
 
-// mode 1: the covariance copy in LDS; 3: in registers (one wave per SIMD,
-// covariate rows staged in LDS where they can be); else re-evaluated
+// mode 1: the covariance copy in LDS; 3: in registers, with what does not fit
+// there in LDS; else re-evaluated
 template <int M>
 static void launch_mixed_m(const BfArgs &a, int variant, int mode,
                            const dim3 &grid, const dim3 &blk, hipStream_t st) {
