@@ -3,22 +3,24 @@
 // (src/util.cpp:261-280) and the site sums the samplers and the conjugate
 // grid need.
 //
-// Two updateBF kernels, both adding up their sites' terms in the same
-// launch (log F_i and e_i e_i^T / F_i, with e_i the residual vector of X
-// and y at site i), so one launch gives everything a Metropolis step or a
-// conjugate grid point needs:
-//  * k_bf_lane<M, COV, BATCH>: one site per lane (64 sites per wavefront),
-//    the whole M x M system in registers, fully unrolled (M <= 16,
-//    closed-form covariances).  Sites with fewer than M neighbors (the
-//    first m sites of the NNGP order) are padded with far-away points:
-//    their rows/columns of C are exactly zero off the diagonal, so the real
-//    block factors bit-for-bit as if unpadded and the padded coefficients
+// The updateBF kernels add up their sites' terms in the same launch (log F_i
+// and e_i e_i^T / F_i, with e_i the residual vector of X and y at site i), so
+// one launch gives everything a Metropolis step or a conjugate grid point
+// needs:
+//  * one site per lane, 64 a wavefront, fully unrolled (M <= 16, closed-form
+//    covariances): k_bf_lane, k_bf_lane_lds (nngp_bf_lane.hpp) and the mixed
+//    k_bf_mixed, k_bf_mixed_reg (nngp_bf_mixed.hip).  Sites with fewer than M
+//    neighbors (the first m sites of the NNGP order) are padded with far-away
+//    points: their rows/columns of C are exactly zero off the diagonal, so the
+//    real block factors bit-for-bit as if unpadded and the padded coefficients
 //    come out exactly 0.  Block size 64, 128 or 256 threads.
-//  * k_bf_coop<BATCH, MM>: one site per wavefront, the matrix built in LDS
-//    and factored with one row per lane in registers (any m <= MM <= 64,
-//    any covariance including the Bessel-K matern),
-//    1, 2 or 4 wavefronts per block walking a contiguous run of sites.
-// Both compute C = s2 R(N,N) + t2 I, c = s2 R(N,i), the Cholesky factor of C
+//  * one site per 16-lane row, four a wavefront (m <= 32, single FP64
+//    problems, any covariance): k_bf_grp (nngp_bf_row.hip).
+//  * k_bf_coop<BATCH, MM> (here): one site per wavefront, the matrix built in
+//    LDS and factored with one row per lane in registers (any m <= MM <= 64,
+//    any covariance including the Bessel-K matern), 1, 2 or 4 wavefronts per
+//    block walking a contiguous run of sites.
+// All compute C = s2 R(N,N) + t2 I, c = s2 R(N,i), the Cholesky factor of C
 // (pivots kept as reciprocal square roots), v = L^-1 c, B = L^-T v and
 // F = s2 + t2 - v.v, i.e. the reference's potrf -> potri -> symv result
 // without forming the inverse.
@@ -458,10 +460,9 @@ bool bf_config_ok(const BfConfig &cfg, int m, int variant) {
 
 // Untuned passes: per lane at 64 threads with finished rows of the factor
 // in LDS where that applies (the fastest per-lane shape at n = 1e6, m = 15);
-// else,
-// for single FP64 problems with m <= 32, the row kernel at 256 threads
-// (n = 4e6, m = 32, Bessel-K matern: 14.8 ms against 41 ms on the
-// wavefront kernel); else the wavefront kernel.
+// else, for single FP64 problems with m <= 32, the row kernel at 256 threads
+// (n = 4e6, m = 32, Bessel-K matern: 11 ms against 41 ms on the wavefront
+// kernel); else the wavefront kernel.
 BfConfig bf_default(int m, int variant, bool single_fp64) {
   BfConfig c;
   if (bf_lane_ok(m, variant)) {

@@ -6,7 +6,8 @@
 // (src/nn.cpp:63-111) does the same by a scan, comparing the Euclidean
 // distances.  The reference walks a u = x + y sorted list; this search uses
 // a strip index (points sorted by x, cut into strips, each strip sorted by
-// y) and one query per lane.  Every pruning test compares a rounded partial
+// y) and one query per wavefront, or per lane for long lists and many nn2
+// queries.  Every pruning test compares a rounded partial
 // square (dx^2 of the strip gap, or dy^2 inside a strip) with the current
 // worst distance; since fl(dx^2) + fl(dy^2) rounds monotonically, nothing
 // that could enter the list is ever skipped, so the result is the exact set
