@@ -56,7 +56,15 @@ __host__ __device__ constexpr int lane_lds_entries(int M) {
 // asm stands behind the finished rows' work by v[k]; it also keeps the kept
 // entries from being held in registers since they were stored, and the loads
 // before it from sinking to their uses.
-template <int M, int K, bool HOOKS, class Entry, class Rhs, class Mid, class Up>
+//
+// EARLY: the pivots' signs are gathered in a scalar mask column by column.
+// Without it the compiler may keep all M pivots and test them where the result
+// is used, M spills: 140 B a lane in kriging at M = 15 (28 with the mask), 28
+// B in the held-out sites and 36 B in the batched updateBF (none).  The single
+// updateBF pass has no spills without the mask and 12 B with it; the spherical
+// kernels over coordinates spill 20% more with it.
+template <int M, int K, bool HOOKS, bool EARLY, class Entry, class Rhs,
+          class Mid, class Up>
 __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,
                                            Rhs &&rhs, double2 *keep,
                                            double (&v)[M], double &vv,
@@ -67,6 +75,7 @@ __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,
   double a[T];  // packed lower triangle, diagonal as 1 / L_jj
   vv = 0.0;
   bool ok = true;
+  unsigned long long pos = ~0ull;
 #pragma unroll
   for (int j = 0; j < M; j++) {
     v[j] = rhs(j);
@@ -82,7 +91,12 @@ __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,
       for (int k = j + 1; k < M; k++)
         a[tri(k, j)] = fma(-a[tri(k, l)], ljl, a[tri(k, j)]);
     }
-    ok = ok && (piv > 0.0);
+    if (EARLY) {
+      pos &= __ballot(piv > 0.0);
+      asm volatile("" : "+s"(pos));
+    } else {
+      ok = ok && (piv > 0.0);
+    }
     const double r = nn_rsqrt(piv);
     a[tri(j, j)] = r;
 #pragma unroll
@@ -119,7 +133,7 @@ __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,
     for (int l = 0; l < k; l++) v[l] = fma(-a[tri(k, l)], t, v[l]);
   }
   if (HOOKS) asm volatile("" : "+v"(v[0]) : : "memory");
-  return ok;
+  return EARLY ? (pos >> (threadIdx.x & 63)) & 1 : ok;
 }
 
 }  // namespace nngp

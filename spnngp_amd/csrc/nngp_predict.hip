@@ -101,7 +101,7 @@ __device__ __forceinline__ double pred_z(const SiteRef &R, int S, int s) {
 // correlation), which leaves the real block's arithmetic unchanged.  The
 // systems are solved at two waves a SIMD (lane_solve): 6,007 sites x 500
 // samples, m = 15, took 760 us with the triangle in registers at one wave;
-// now 578 us.
+// now 486 us.
 template <int M, int COV>
 __global__ __launch_bounds__(kPredLane, 2) void k_pred_lane(PredArgs A) {
   constexpr int K = lane_lds_entries(M);
@@ -158,7 +158,7 @@ __global__ __launch_bounds__(kPredLane, 2) void k_pred_lane(PredArgs A) {
   const double nug = latent ? 0.0 : t2;
   double v[M];  // w
   double vv;
-  const bool ok = lane_solve<M, K, false>(
+  const bool ok = lane_solve<M, K, false, true>(
       s2 * 1.0 + nug,
       [&](int k, int l) {
         return s2 *

@@ -46,3 +46,49 @@ def test_rows_in_lds_match_the_oracle(oracle, nngp, m, p, cov, theta):
             r = X @ beta - y
             q0 = oracle.Q(B0, F0, r, r, nn["nnIndx"], lu)
             assert abs(out["qResid"] - q0) < RTOL * abs(q0)
+
+
+# The solve's verdict reaches the caller from a lane of a partly filled second
+# wave: sample 70 of 77 alone has no nugget, and the new site's two nearest
+# neighbors coincide, so its second pivot is exactly 4 - 2 * 2 = 0.
+@pytest.mark.parametrize("m", [10, 15, 16])
+@pytest.mark.parametrize("cov", [0, 1, 3])
+def test_kriging_reports_the_one_singular_sample(nngp, m, cov):
+    n, S, q = 400, 77, 3
+    c = uniform_coords(n, 77 + m)
+    rng = np.random.default_rng(m)
+    c[201] = c[200]
+    X = np.ones((n, 1))
+    y = rng.normal(size=n)
+    c0 = c[[50, 200, 300]] + 1e-6
+    nn0 = np.array([np.argsort(((c - s) ** 2).sum(1), kind="stable")[:m]
+                    for s in c0])
+    assert set(nn0[1, :2]) == {200, 201}
+    theta = np.repeat([[4.0], [0.5], [3.0]], S, axis=1)
+    beta = np.zeros((1, S))
+    z = rng.normal(size=q * S)
+    args = (X, y, c, n, 1, m, np.ones((q, 1)), c0, q, nn0, beta)
+    ok = nngp.rNNGPPredict(*args, theta, S, cov, z=z)["p.y.0"]
+    assert np.isfinite(ok).all()
+    theta[1, 70] = 0.0
+    with pytest.raises(nngp.NngpError) as e:
+        nngp.rNNGPPredict(*args, theta, S, cov, z=z)
+    assert e.value.status == nngp.NNGP_ERR_NOT_PD
+
+
+@pytest.mark.parametrize("cov,tail", [(0, []), (1, []), (2, [1.5]), (3, [])])
+def test_grid_reports_a_singular_training_site(nngp, cov, tail):
+    """A training site whose two nearest neighbors coincide: alpha = 0 is
+    singular there, alpha = 0.1 is not."""
+    n, m = 500, 15
+    c = uniform_coords(n, 31)
+    c[201] = c[200]
+    c[202] = c[200] + 1e-6
+    rng = np.random.default_rng(5)
+    ho = np.array([np.arange(0, 40), np.arange(400, 440)])
+    with nngp.CvGrid(rng.normal(size=n), np.ones((n, 1)), c, m, ho,
+                     [2.0, 1.0], cov, shape=(0, 64, 2)) as g:
+        assert np.isfinite(g.run([[3.0, 0.1] + tail])["scores"]).all()
+        with pytest.raises(nngp.NngpError) as e:
+            g.run([[3.0, 0.1] + tail, [3.0, 0.0] + tail])
+        assert e.value.status == nngp.NNGP_ERR_NOT_PD
