@@ -885,11 +885,15 @@ __device__ inline float s2_corr32_rt(float d2, const CovArgs32 &a,
 // false when a pivot is not positive.
 template <int M>
 __device__ __forceinline__ bool chol_factor32(float (&a)[M * (M + 1) / 2]) {
-  bool ok = true;
+  // the pivots' signs in a scalar mask, column by column: tested after the
+  // solve, the M pivots would be held or spilled until then (at M = 15 44 B a
+  // lane in k_bf_mixed_reg; now none)
+  unsigned long long pos = ~0ull;
 #pragma unroll
   for (int j = 0; j < M; j++) {
     const float piv = a[tri(j, j)];
-    ok = ok && (piv > 0.0f);
+    pos &= __ballot(piv > 0.0f);
+    asm volatile("" : "+s"(pos));
     const float r = __builtin_amdgcn_rsqf(piv);
     a[tri(j, j)] = r;
 #pragma unroll
@@ -902,7 +906,7 @@ __device__ __forceinline__ bool chol_factor32(float (&a)[M * (M + 1) / 2]) {
         a[tri(k, l)] = fmaf(-lkj, a[tri(l, j)], a[tri(k, l)]);
     }
   }
-  return ok;
+  return (pos >> (threadIdx.x & 63)) & 1;
 }
 
 // v <- C^-1 v with the factor of chol_factor32.
