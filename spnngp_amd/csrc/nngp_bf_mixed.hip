@@ -201,7 +201,7 @@ __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed(BfArgs A) {
 // step, so B and F equal its results bit for bit.  With the whole copy in
 // registers, one wave per SIMD and the covariate rows staged in LDS, a pass
 // took 155 us at n = 1e6, m = 15 (the vector units busy 61% of the time);
-// now 120 us.  ZH > 0: the rows of Z are ZH aligned pairs.
+// now 104 us.  ZH > 0: the rows of Z are ZH aligned pairs.
 __host__ __device__ constexpr int mixed_lds_entries(int M) {
   return M <= 12 ? 0 : 72;
 }
