@@ -402,9 +402,30 @@ __device__ __forceinline__ WaveList wave_search(const StripIndex &S, int t0,
   return L;
 }
 
-__global__ __launch_bounds__(kKnnBlock) void k_nn2_wave(Nn2Args A) {
-  const int i = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * kKnnBlock + threadIdx.x) >> 6));
+// Queries of one launch, a wavefront each: a grid holds fewer than 2^32
+// threads, so 2^26 queries and more do not fit one.
+constexpr int kWaveQueries = 1 << 25;
+constexpr int kWaveBlock = kKnnBlock / 64;  // queries a block
+
+// launch(first, blocks) for each launch over n queries
+template <class Launch>
+static int wave_launches(int n, Launch launch) {
+  for (long long first = 0; first < n; first += kWaveQueries) {
+    const int left = (int)std::min<long long>(n - first, kWaveQueries);
+    launch((int)first, dim3((left + kWaveBlock - 1) / kWaveBlock));
+    if (const hipError_t e = hipGetLastError()) return (int)e;
+  }
+  return 0;
+}
+
+// The wavefront's query, of those from `first` on.
+__device__ __forceinline__ int wave_query(int first) {
+  return first + (int)blockIdx.x * kWaveBlock +
+         __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
+}
+
+__global__ __launch_bounds__(kKnnBlock) void k_nn2_wave(Nn2Args A, int first) {
+  const int i = wave_query(first);
   const int t = (int)threadIdx.x & 63;
   if (i >= A.nq) return;
   const double2 q = A.q[i];
@@ -423,9 +444,9 @@ __global__ __launch_bounds__(kKnnBlock) void k_nn2_wave(Nn2Args A) {
 // n = 1e6, m = 15: 9.6 ms with one lane a site, whose every accepted candidate
 // moves a 16-entry list of all 64 lanes; now 3.4 ms.  n = 5e5 clustered, m =
 // 32: 9.7 and 2.7 ms.
-__global__ __launch_bounds__(kKnnBlock) void k_knn_pred_wave(KnnArgs A) {
-  const int i = __builtin_amdgcn_readfirstlane(
-      (int)((blockIdx.x * kKnnBlock + threadIdx.x) >> 6));
+__global__ __launch_bounds__(kKnnBlock) void k_knn_pred_wave(KnnArgs A,
+                                                            int first) {
+  const int i = wave_query(first);
   const int t = (int)threadIdx.x & 63;
   if (i >= A.n) return;
   int off, cnt;
@@ -463,8 +484,10 @@ __global__ __launch_bounds__(kKnnBlock) void k_knn_pred_wave(KnnArgs A) {
 int knn_launch(const KnnArgs &a, hipStream_t st) {
   const dim3 block(kKnnBlock);
   if (a.m < 64)
-    hipLaunchKernelGGL(k_knn_pred_wave, dim3((a.n + 3) / 4), block, 0, st, a);
-  else if (a.m < 65)  // 65 candidates: one site a lane
+    return wave_launches(a.n, [&](int first, dim3 grid) {
+      hipLaunchKernelGGL(k_knn_pred_wave, grid, block, 0, st, a, first);
+    });
+  if (a.m < 65)  // 65 candidates: one site a lane
     hipLaunchKernelGGL(k_knn_pred<65>, dim3((a.n + kKnnBlock - 1) / kKnnBlock),
                        block, 0, st, a);
   else
@@ -738,10 +761,11 @@ int nn2_launch(const Nn2Args &a, hipStream_t st) {
   if (a.k > 64) return -1;
   const dim3 block(kKnnBlock);
   if (a.k > 16 || a.nq <= kNn2Wave)
-    hipLaunchKernelGGL(k_nn2_wave, dim3((a.nq + 3) / 4), block, 0, st, a);
-  else
-    hipLaunchKernelGGL(k_nn2<16>, dim3((a.nq + kKnnBlock - 1) / kKnnBlock),
-                       block, 0, st, a);
+    return wave_launches(a.nq, [&](int first, dim3 grid) {
+      hipLaunchKernelGGL(k_nn2_wave, grid, block, 0, st, a, first);
+    });
+  hipLaunchKernelGGL(k_nn2<16>, dim3((a.nq + kKnnBlock - 1) / kKnnBlock), block,
+                     0, st, a);
   return (int)hipGetLastError();
 }
 

@@ -33,3 +33,33 @@ def test_nn2_bit_exact(oracle, nngp, n, k, q):
     i_ref, d_ref = oracle.nn2(c, c0, k)
     i_got, d_got = nngp.nn2(c, c0, k)
     assert np.array_equal(i_got, i_ref) and np.array_equal(d_got, d_ref)
+
+
+def test_more_sites_than_one_launch_holds(nngp):
+    """2^26 + 5 sites, m = 1: one grid of a wavefront a site would be 2^32
+    threads and more.  Sites in pairs 2k, 2k + 1 at (k, y_k) and
+    (k + 1/4, y_k), y random: an odd site's nearest predecessor is its twin, as
+    every other site is at least 3/4 off in x.  Even sites at both ends and on
+    both sides of 2^25 and 2^26 are checked by hand."""
+    n = (1 << 26) + 5
+    print(f"knn n={n} m=1", flush=True)
+    i = np.arange(n, dtype=np.int32)
+    c = np.empty((n, 2), order="F")
+    c[:, 0] = (i >> 1) + 0.25 * (i & 1)
+    y = np.random.default_rng(7).uniform(0.0, 8192.0, (n + 1) // 2)
+    c[:, 1] = y[i >> 1]
+    got = nngp.mkNNIndx(c, 1)
+    idx, dist = got["nnIndx"], got["nnDist"]
+    lu = got["nnIndxLU"]
+    assert np.array_equal(lu[1:n], i[:-1]) and lu[0] == 0
+    assert lu[n] == 0 and (lu[n + 1:] == 1).all()
+    assert idx.size == n - 1  # entry s - 1 is site s's
+    assert np.array_equal(idx[0::2], i[0:n - 1:2])
+    assert (dist[0::2] == 0.25).all()
+    for s in [2, 4, 100, n - 3, n - 1] + [
+            b + d for b in (1 << 25, 1 << 26) for d in (-2, 0, 2)]:
+        lo = max(0, s - 200000)  # farther than 8192 in x
+        d = np.hypot(c[lo:s, 0] - c[s, 0], c[lo:s, 1] - c[s, 1])
+        k = int(np.argmin(d))
+        assert idx[s - 1] == lo + k, s
+        assert abs(dist[s - 1] - d[k]) <= 1e-12 * d[k], s
