@@ -416,12 +416,15 @@ typedef struct nngp_tune_report {
   int mode[NNGP_TUNE_MAX];        /* family 0, NNGP_MIXED: 1 = the
                                      covariance copy kept in LDS for the
                                      refinement residual, 3 = kept in
-                                     registers (one wave per SIMD), 0 =
-                                     re-evaluated; family 0, FP64:
+                                     registers and LDS (two waves per
+                                     SIMD), 0 = re-evaluated; family 0, FP64:
                                      2 = finished rows of the factor kept
                                      in LDS, two waves per SIMD (same
                                      results bit for bit as 0)            */
-  double ms[NNGP_TUNE_MAX];       /* mean launch time                     */
+  double ms[NNGP_TUNE_MAX];       /* mean of three launches; of a shape at
+                                     half another's speed one launch, in a
+                                     grid of a sixteenth of the problems and
+                                     scaled to all of them                */
   int best_family, best_threads, best_mode;
 } nngp_tune_report;
 

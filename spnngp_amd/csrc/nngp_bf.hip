@@ -39,9 +39,6 @@
 #include <algorithm>
 #include <climits>
 #include <cstdint>
-#include <map>
-#include <mutex>
-#include <tuple>
 #include <vector>
 
 #include "nngp_bf.hpp"
@@ -592,29 +589,12 @@ int bf_sums_launch(const BfArgs &a, const BfConfig &cfg, int nprob,
 // ---------------------------------------------------------------------------
 // Candidates: sites per wavefront (64: the per-lane kernel at 64, 128 or
 // 256 threads per block; 1: the wavefront kernel with 1, 2 or 4 waves per
-// block, i.e. LDS tiles of 1, 2 or 4 systems).  Each is timed with HIP
-// events on the caller's stream (one warm-up, then three launches; fewer
-// where it is far behind) and the fastest kept.  Results are cached per (m, variant, nz, size class).
-namespace {
-std::mutex g_tune_mu;
-std::map<std::tuple<int, int, int, int>, BfConfig> g_tune_cache;
-}  // namespace
-
+// block, i.e. LDS tiles of 1, 2 or 4 systems; 4: the row kernel).  Each is
+// timed with HIP events on the caller's stream (one warm-up, then three
+// launches; fewer where it is far behind) and the fastest kept.
 int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
                 BfTuneReport *rep) {
   const int variant = a.variant;
-  const long long work = (long long)a.n * nprob;
-  int cls = 0;
-  while ((1LL << (cls + 1)) <= work) cls++;
-  const auto key = std::make_tuple(a.m, variant * 4 + a.mixed, a.nz, cls);
-  if (!rep) {
-    std::lock_guard<std::mutex> lk(g_tune_mu);
-    auto it = g_tune_cache.find(key);
-    if (it != g_tune_cache.end()) {
-      *best = it->second;
-      return 0;
-    }
-  }
   std::vector<BfConfig> cand;
   if (a.mixed) {  // the per-lane mixed kernel: block size x covariance
                   // copy (none, LDS, registers); then the wavefront one
@@ -656,12 +636,16 @@ int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
     if (a.rows && bf_rows(a, cfg) > a.rows_cap) continue;
     double per = 0.0;
     // a candidate that a sixteenth of the problems (or the one problem) shows
-    // to be half as fast as another is not timed further: the wavefront shapes
-    // of a 250-problem grid cost 370 of its first run's 393 ms
+    // to be half as fast as one before it is not timed further, nor kept; its
+    // report is that one launch's time scaled to all problems.  The wavefront
+    // shapes of a 250-problem grid cost 370 of its first run's 393 ms.  Few
+    // problems leave part of the chip idle, which favors the shapes with more
+    // waves; those stand behind the per-lane ones, so none is ruled out by it.
     const int few = std::max(1, nprob / 16);
     if ((rc = timed(cfg, few, 1, &per)) != 0) break;
     best_few = std::min(best_few, per);
-    if (per < 2.0 * best_few)
+    const bool whole = per < 2.0 * best_few;
+    if (whole)
       rc = timed(cfg, nprob, 3, &per);
     else
       per *= (double)nprob / few;
@@ -673,7 +657,7 @@ int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
       rep->ms[nc] = per;
     }
     nc++;
-    if (per < best_ms) {
+    if (whole && per < best_ms) {
       best_ms = per;
       pick = cfg;
     }
@@ -686,8 +670,6 @@ int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
     rep->best = pick;
     rep->best_ms = best_ms;
   }
-  std::lock_guard<std::mutex> lk(g_tune_mu);
-  g_tune_cache[key] = pick;
   *best = pick;
   return 0;
 }

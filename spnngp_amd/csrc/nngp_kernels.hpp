@@ -133,8 +133,8 @@ int rows_sum_launch(const double *rows, int cap, int nrows, long long ps_rows,
                     int nv, int nprob, double *out, int out_stride, int *err,
                     double *err_out, hipStream_t st,
                     const SumsSignal *sig = nullptr);
-// Time every applicable launch shape of this pass and keep the fastest
-// (cached per (m, variant, nz, size class) unless rep asks for timings).
+// Time every applicable launch shape of this pass and keep the fastest; rep
+// may be nullptr.
 int bf_autotune(const BfArgs &a, int nprob, hipStream_t st, BfConfig *best,
                 BfTuneReport *rep);
 int q_launch(const QArgs &a, hipStream_t st);

@@ -131,8 +131,8 @@ def test_cvgrid_autotuner_reports_candidates(nngp):
         r = cv.run(ta)
     tune = r["tune"]
     kinds = {t[0] for t in tune}
-    # per lane at 64/128/256 threads, staged at 64/128 (256 would need
-    # 128 KiB of LDS a block), per wavefront at 1/2/4 waves
+    # per lane at 64/128/256 threads, with finished rows in LDS at 64/128
+    # (256 would need 72 KiB a block), per wavefront at 1/2/4 waves
     assert kinds == {"lane", "lane+lds-z", "wave"} and len(tune) == 8
     best = min(tune, key=lambda t: t[2])
     assert r["bf_config"] == (best[0], best[1])
