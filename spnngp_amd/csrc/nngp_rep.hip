@@ -19,7 +19,7 @@
 //    shim) they are drawn on the host in the reference's order, all n of
 //    sample s before sample s + 1, so the replicates follow R's stream.
 //    Without one they are counter-based Philox normals keyed by
-//    (seed, site, sample), drawn in the kernel.
+//    (seed, site, sample), drawn by k_rep_noise.
 #include <algorithm>
 #include <climits>
 #include <cstdio>

@@ -141,6 +141,38 @@ def test_replicates_in_three_groups_reuse_the_output_buffers(oracle, nngp):
         assert rel(got[:, s], want[:, 0]) < RTOL
 
 
+def level_widths(n, nn):
+    idx, lu = nn["nnIndx"], nn["nnIndxLU"]
+    lev = np.zeros(n, int)
+    for i in range(1, n):
+        lev[i] = 1 + lev[idx[lu[i]:lu[i] + lu[n + i]]].max()
+    return np.bincount(lev)
+
+
+@pytest.mark.parametrize("n,m,lo,hi", [
+    (2500, 12, 65, 128),      # 128-thread blocks
+    (6000, 8, 129, 256),      # 256
+    (12000, 8, 257, 1 << 30),  # 256, levels of two passes
+    (20000, 16, 257, 1 << 30)])
+def test_replicates_with_wide_levels(oracle, nngp, n, m, lo, hi):
+    """Sites in random order have wide dependency levels: blocks of several
+    waves (a level's values cross them at the barrier) and levels with more
+    sites than the block has threads.  The x-ordered sites above stay within
+    64 a level, one wave."""
+    p, S = 2, 3
+    print(f"rep wide levels n={n} m={m}", flush=True)
+    c, X, beta, th = problem(n, m, p, S, 0, 50 + m)
+    c = np.random.default_rng(n).permutation(c)
+    nn = oracle.mkNNIndxCB(c, m)
+    assert lo <= level_widths(n, nn).max() <= hi
+    z = np.random.default_rng(3).normal(size=n * S)
+    want = oracle_rep(oracle, c, X, beta, th, nn, m, 0, z)
+    got = nngp.rNNGPReplicated(X, p, n, m, c, 0, nn["nnIndx"],
+                               nn["nnIndxLU"], beta, th, S,
+                               rng=oracle.TapeRng(z, []))["y.rep.samples"]
+    assert rel(got, want) < RTOL
+
+
 def test_replicates_reject_a_neighbor_that_is_not_a_predecessor(oracle,
                                                                  nngp):
     n, m, p, S = 200, 4, 1, 2
