@@ -78,7 +78,7 @@ __device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
   double2 z[ZH > 0 ? ZH : 1], zn[ZH > 0 ? M * ZH : 1];
   double v[M];  // B_i
   double vv;
-  const bool ok = lane_solve<M, K, (ZH > 0), BATCH && COV != 1>(
+  const bool ok = lane_solve<M, K, (ZH > 0), (BATCH || M > 15)>(
       c.diag,
       [&](int k, int l) {
         return lane_corr<COV>(lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);

@@ -252,7 +252,7 @@ __global__ __launch_bounds__(kCvPredThreads, 2) void k_cv_pred_lane(
     }
     double v[M];  // w
     double vv;
-    const bool ok = lane_solve<M, K, true, COV != 1>(
+    const bool ok = lane_solve<M, K, true, true>(
         c.diag,
         [&](int k, int l) {
           return lane_corr<COV>(lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);

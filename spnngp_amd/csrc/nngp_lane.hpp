@@ -61,8 +61,9 @@ __host__ __device__ constexpr int lane_lds_entries(int M) {
 // Without it the compiler may keep all M pivots and test them where the result
 // is used, M spills: 140 B a lane in kriging at M = 15 (28 with the mask), 28
 // B in the held-out sites and 36 B in the batched updateBF (none).  The single
-// updateBF pass has no spills without the mask and 12 B with it; the spherical
-// kernels over coordinates spill 20% more with it.
+// updateBF pass at M = 15 has no spills without the mask and 12 B with it; at M
+// = 16 84 to 172 B without and 0 to 44 B with it (n = 3,000, p = 3, exponential:
+// 17.1 us, now 15.8; n = 1e6 241 and 210).
 template <int M, int K, bool HOOKS, bool EARLY, class Entry, class Rhs,
           class Mid, class Up>
 __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,

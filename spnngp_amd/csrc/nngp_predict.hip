@@ -37,9 +37,8 @@ __device__ __forceinline__ double corr_d(double D, double phi, double ip,
   if constexpr (COV == 0) {
     return s2_exp2(-phs * D, u);  // exp(-phi D) = 2^(-phi D / ln 2)
   } else if constexpr (COV == 1) {
-    const double t = phi * D;
-    const double v = 1.0 - 1.5 * t + 0.5 * (t * t * t);
-    return (D > 0.0 && D <= ip) ? v : (D >= ip ? 0.0 : 1.0);
+    const double t = D <= ip ? phi * D : (D >= ip ? 1.0 : 0.0);
+    return 1.0 - 1.5 * t + 0.5 * (t * t * t);
   } else {
     const double t = phs * D;  // phi D / sqrt(ln 2)
     return s2_exp2(-(t * t), u);

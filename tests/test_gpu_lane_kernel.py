@@ -92,3 +92,31 @@ def test_grid_reports_a_singular_training_site(nngp, cov, tail):
         with pytest.raises(nngp.NngpError) as e:
             g.run([[3.0, 0.1] + tail, [3.0, 0.0] + tail])
         assert e.value.status == nngp.NNGP_ERR_NOT_PD
+
+
+# The spherical is one formula of a selected argument: 0 beyond the range, the
+# sill at distance 0.  On a lattice of spacing 1/8 with a range of 1/4 and
+# doubled sites the distances 0 and exactly 1/phi both occur.
+@pytest.mark.parametrize("m,shape", [(4, (0, 64, 0)), (15, (0, 64, 2)),
+                                     (16, (0, 64, 2)), (16, (0, 256, 0)),
+                                     (20, (2, 256, 0)), (40, (1, 64, 0))])
+def test_spherical_at_its_edges(oracle, nngp, m, shape):
+    print(f"spherical edges m={m} shape={shape}", flush=True)
+    g = np.arange(18) / 8.0
+    c = np.array([(x, y) for x in g for y in g])
+    rng = np.random.default_rng(m)
+    c = np.vstack([c, c[rng.integers(0, len(c), 60)]])
+    c = c[np.argsort(c[:, 0], kind="stable")]
+    n = len(c)
+    nn = oracle.mkNNIndxCB(c, m)
+    theta = [1.5, 0.3, 4.0]
+    B0, F0, ld0 = oracle.updateBF(c.T.reshape(-1).copy(), nn["nnIndx"],
+                                  nn["nnIndxLU"], n, m, theta, 1)
+    X, y = np.ones((n, 1)), rng.normal(size=n)
+    with nngp.Model(c, nn["nnIndx"], nn["nnIndxLU"], m, 1, X, y) as md:
+        md.set_shape(*shape)
+        out = md.update(theta, slot=0, beta=np.zeros(1))
+        B, F = md.get_bf(0)
+    assert np.max(np.abs(F - F0) / F0) < RTOL
+    assert np.max(np.abs(B - B0)) < RTOL * np.max(np.abs(B0))
+    assert abs(out["logDet"] - ld0) < RTOL * max(abs(ld0), 1.0)
