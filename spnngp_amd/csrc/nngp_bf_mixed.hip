@@ -195,24 +195,34 @@ __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed(BfArgs A) {
 }
 
 // k_bf_mixed's scheme with a copy of C kept, so that no entry is evaluated
-// twice: what of the copy the registers of two waves per SIMD cannot hold
+// twice: what of the copy the registers of W = 2 waves per SIMD cannot hold
 // beside the factor waits in LDS for the residual (mixed_lds_entries, four
 // entries a lane in each 16 bytes).  The arithmetic is k_bf_mixed's step for
 // step, so B and F equal its results bit for bit.  With the whole copy in
 // registers, one wave per SIMD and the covariate rows staged in LDS, a pass
 // took 155 us at n = 1e6, m = 15 (the vector units busy 61% of the time);
 // now 104 us.  ZH > 0: the rows of Z are ZH aligned pairs.
-__host__ __device__ constexpr int mixed_lds_entries(int M) {
-  return M <= 12 ? 0 : 72;
+//
+// At M = 16 two waves lack 29 registers (43 to 54 with the spherical's former
+// branches), and LDS has no room for them.  With W = 1 nothing spills and
+// the covariate rows can be requested with the coordinates.  W = 2 and 1, p =
+// 3, exponential: n = 3,000 15.2 and 12.6 us, n = 2e5 45.2 and 43.7, n = 1e6
+// 185 and 179.  Rows that are not pairs come after the solve, where a second
+// wave covers their wait as soon as there is one (launch_mixed_reg_mh).
+__host__ __device__ constexpr int mixed_lds_entries(int M, int W) {
+  return M <= 12 || W == 1 ? 0 : 72;
 }
 
-template <int M, int COV, int ZH>
+template <int M, int COV, int ZH, int W>
 __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
                                                int cnt, int off,
                                                int (&nb)[M], double &Fi,
                                                double (&e)[kMaxNZ],
                                                float4 *keep) {
-  constexpr int K = mixed_lds_entries(M);
+  constexpr int K = mixed_lds_entries(M, W);
+  constexpr bool kEarlyZ = ZH > 0 && W == 1;
+  const double2 *Z = reinterpret_cast<const double2 *>(A.Z);
+  double2 z[ZH > 0 ? ZH : 1], zn[kEarlyZ ? M * ZH : 1];
   const CovArgs &c = A.c;
   const CovArgs32 c32 = cov32(c);
   if (cnt == 0) {  // site 0: F = s2 + t2, residual = the data
@@ -234,6 +244,16 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
     const double2 q = A.xy[nb[k]];
     dx[k] = (float)(q.x - s.x);
     dy[k] = (float)(q.y - s.y);
+  }
+  if constexpr (kEarlyZ) {
+#pragma unroll
+    for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
+#pragma unroll
+    for (int k = 0; k < M; k++) {
+#pragma unroll
+      for (int h = 0; h < ZH; h++) zn[k * ZH + h] = Z[(size_t)nb[k] * ZH + h];
+    }
+    asm volatile("" : : : "memory");
   }
   if (cnt < M) {  // far away and far apart: correlations exactly 0
 #pragma unroll
@@ -290,9 +310,11 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
     }
   }
   // the neighbor slots again (from cache), in time for the covariate rows
-  asm volatile("" : "+v"(r[0]) : : "memory");
+  if constexpr (!kEarlyZ) {
+    asm volatile("" : "+v"(r[0]) : : "memory");
 #pragma unroll
-  for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
+    for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
+  }
   float d[M];
 #pragma unroll
   for (int k = 0; k < M; k++) d[k] = (float)r[k];
@@ -314,15 +336,17 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
 #pragma unroll
   for (int k = 0; k < M; k++) nb[k] = k < cnt ? nb[k] : 0;
   if constexpr (ZH > 0) {
-    const double2 *Z = reinterpret_cast<const double2 *>(A.Z);
-    double2 z[ZH];
+    if constexpr (!kEarlyZ) {
 #pragma unroll
-    for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
+      for (int h = 0; h < ZH; h++) z[h] = Z[(size_t)i * ZH + h];
+    }
 #pragma unroll
     for (int k = 0; k < M; k++) {
 #pragma unroll
       for (int h = 0; h < ZH; h++) {
-        const double2 q = Z[(size_t)nb[k] * ZH + h];
+        double2 q;
+        if constexpr (kEarlyZ) q = zn[k * ZH + h];
+        else q = Z[(size_t)nb[k] * ZH + h];
         z[h].x = fma(-bd[k], q.x, z[h].x);
         z[h].y = fma(-bd[k], q.y, z[h].y);
       }
@@ -349,22 +373,23 @@ __device__ __forceinline__ void mixed_reg_site(const BfArgs &A, int i,
 
 // Dynamic LDS of k_bf_mixed_reg a wavefront, in double2: the kept entries,
 // which the block sums then overwrite, or the sums' terms.
-__host__ __device__ inline int mixed_reg_wave_chunks(int M, int nz) {
+__host__ __device__ inline int mixed_reg_wave_chunks(int M, int W, int nz) {
   const int sums = (site_terms(nz) * 64 + 1) / 2;
-  const int keep = mixed_lds_entries(M) / 4 * 64;
+  const int keep = mixed_lds_entries(M, W) / 4 * 64;
   return keep > sums ? keep : sums;
 }
 
-template <int M, int COV, int ZH>
-__global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed_reg(BfArgs A) {
-  extern __shared__ double2 mstage[];
+// The body of both register-copy kernels; mstage: the block's dynamic LDS.
+template <int M, int COV, int ZH, int W>
+__device__ __forceinline__ void mixed_reg_body(const BfArgs &A,
+                                               double2 *mstage) {
   const int nt = (int)blockDim.x;
   const int b = xcd_block((A.n + nt - 1) / nt);
   if (b < 0) return;  // whole padding block
   const int i = b * nt + (int)threadIdx.x;
   const bool valid = i < A.n;
   const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
-  double2 *stg = mstage + (size_t)w * mixed_reg_wave_chunks(M, A.nz);
+  double2 *stg = mstage + (size_t)w * mixed_reg_wave_chunks(M, W, A.nz);
   double Fi = 1.0;
   double e[kMaxNZ];
 #pragma unroll
@@ -380,7 +405,7 @@ __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed_reg(BfArgs A) {
     int nb[M];
 #pragma unroll
     for (int k = 0; k < M; k++) nb[k] = A.nnIndx[off + k];
-    mixed_reg_site<M, COV, ZH>(
+    mixed_reg_site<M, COV, ZH, W>(
         A, i, cnt, off, nb, Fi, e,
         reinterpret_cast<float4 *>(stg) + ((int)threadIdx.x & 63));
     if (A.F) A.F[i] = Fi;
@@ -388,6 +413,18 @@ __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed_reg(BfArgs A) {
   if (A.rows)
     block_site_terms_lds(A.nz, A.rows, A.rows_cap, valid, Fi, e, b,
                          reinterpret_cast<double *>(stg));
+}
+
+template <int M, int COV, int ZH>
+__global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_mixed_reg(BfArgs A) {
+  extern __shared__ double2 mixed_lds[];
+  mixed_reg_body<M, COV, ZH, 2>(A, mixed_lds);
+}
+
+template <int M, int COV, int ZH>
+__global__ __launch_bounds__(kLaneMaxThreads, 1) void k_bf_mixed_one(BfArgs A) {
+  extern __shared__ double2 mixed_lds[];
+  mixed_reg_body<M, COV, ZH, 1>(A, mixed_lds);
 }
 
 // LDS of the mixed kernel's covariance copy: (M(M+1)/2 + M) floats a lane.
@@ -415,38 +452,64 @@ static void launch_mixed_mc(const BfArgs &a, int variant, const dim3 &grid,
 }
 
 // Aligned pairs in a row of Z that k_bf_mixed_reg reads (zs = 2 ZH, Z 16-byte
-// aligned, m > 8), else 0: single values, as also for rows of two pairs in
-// 256-thread blocks, a shape that smaller blocks beat.
-static int mixed_reg_zh(const BfArgs &a, int threads) {
+// aligned, m > 8), else 0: single values.
+static int mixed_reg_zh(const BfArgs &a) {
   if (!a.Z || a.nz <= 0 || a.m <= 8 || ((uintptr_t)a.Z & 15) != 0) return 0;
-  return a.zs == 2 ? 1 : a.zs == 4 && threads <= 128 ? 2 : 0;
+  return a.zs == 2 ? 1 : a.zs == 4 ? 2 : 0;
 }
 
-static size_t mixed_reg_shm(const BfArgs &a, int threads) {
-  return (size_t)(threads / 64) * mixed_reg_wave_chunks(lane_M(a.m), a.nz) *
-         sizeof(double2);
+// Sites up to which no SIMD of the 1,024 has a second wave.
+constexpr int kOneWaveSites = 1024 * 64;
+
+template <int M, int ZH, int W>
+static void launch_mixed_reg_mhw(const BfArgs &a, int variant,
+                                 const dim3 &grid, const dim3 &blk,
+                                 hipStream_t st) {
+  const size_t shm = (size_t)(blk.x / 64) *
+                     mixed_reg_wave_chunks(M, W, a.nz) * sizeof(double2);
+  auto launch = [&](auto cov) {
+    constexpr int COV = decltype(cov)::value;
+    if constexpr (W == 2)
+      hipLaunchKernelGGL((k_bf_mixed_reg<M, COV, ZH>), grid, blk, shm, st, a);
+    else
+      hipLaunchKernelGGL((k_bf_mixed_one<M, COV, ZH>), grid, blk, shm, st, a);
+  };
+  switch (variant) {
+    case 0: launch(std::integral_constant<int, 0>()); break;
+    case 1: launch(std::integral_constant<int, 1>()); break;
+    case kCovMatern15:
+      launch(std::integral_constant<int, kCovMatern15>());
+      break;
+    case kCovMatern25:
+      launch(std::integral_constant<int, kCovMatern25>());
+      break;
+    default: launch(std::integral_constant<int, 3>()); break;
+  }
 }
 
+// W = 2 up to M = 15, where everything fits; at M = 16 W = 1, but for rows of
+// Z that are not pairs only while no SIMD has two waves (p = 5, W = 2 and 1: n
+// = 3,000 15.1 and 14.4 us, n = 70,000 33.0 and 38.5).
 template <int M, int ZH>
 static void launch_mixed_reg_mh(const BfArgs &a, int variant, const dim3 &grid,
-                                const dim3 &blk, size_t shm, hipStream_t st) {
-  switch (variant) {
-    case 0: hipLaunchKernelGGL((k_bf_mixed_reg<M, 0, ZH>), grid, blk, shm, st, a); break;
-    case 1: hipLaunchKernelGGL((k_bf_mixed_reg<M, 1, ZH>), grid, blk, shm, st, a); break;
-    case kCovMatern15: hipLaunchKernelGGL((k_bf_mixed_reg<M, kCovMatern15, ZH>), grid, blk, shm, st, a); break;
-    case kCovMatern25: hipLaunchKernelGGL((k_bf_mixed_reg<M, kCovMatern25, ZH>), grid, blk, shm, st, a); break;
-    default: hipLaunchKernelGGL((k_bf_mixed_reg<M, 3, ZH>), grid, blk, shm, st, a); break;
+                                const dim3 &blk, hipStream_t st) {
+  if constexpr (M <= 15) {
+    launch_mixed_reg_mhw<M, ZH, 2>(a, variant, grid, blk, st);
+  } else {
+    if (ZH == 0 && a.n > kOneWaveSites)
+      launch_mixed_reg_mhw<M, 0, 2>(a, variant, grid, blk, st);
+    else
+      launch_mixed_reg_mhw<M, ZH, 1>(a, variant, grid, blk, st);
   }
 }
 
 template <int M>
 static void launch_mixed_reg(const BfArgs &a, int variant, const dim3 &grid,
                              const dim3 &blk, hipStream_t st) {
-  const size_t shm = mixed_reg_shm(a, (int)blk.x);
-  switch (mixed_reg_zh(a, (int)blk.x)) {
-    case 1: launch_mixed_reg_mh<M, 1>(a, variant, grid, blk, shm, st); break;
-    case 2: launch_mixed_reg_mh<M, 2>(a, variant, grid, blk, shm, st); break;
-    default: launch_mixed_reg_mh<M, 0>(a, variant, grid, blk, shm, st); break;
+  switch (mixed_reg_zh(a)) {
+    case 1: launch_mixed_reg_mh<M, 1>(a, variant, grid, blk, st); break;
+    case 2: launch_mixed_reg_mh<M, 2>(a, variant, grid, blk, st); break;
+    default: launch_mixed_reg_mh<M, 0>(a, variant, grid, blk, st); break;
   }
 }
 

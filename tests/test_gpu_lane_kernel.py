@@ -120,3 +120,34 @@ def test_spherical_at_its_edges(oracle, nngp, m, shape):
     assert np.max(np.abs(F - F0) / F0) < RTOL
     assert np.max(np.abs(B - B0)) < RTOL * np.max(np.abs(B0))
     assert abs(out["logDet"] - ld0) < RTOL * max(abs(ld0), 1.0)
+
+
+@pytest.mark.parametrize("cov,n,p", [(0, 4013, 1), (1, 4013, 3), (2, 4013, 5),
+                                     (0, 65536, 5), (1, 65537, 5),
+                                     (2, 65601, 3)])
+def test_mixed_m16_forms_agree(nngp, cov, n, p):
+    """m = 16 in mixed precision: the form with the covariance in registers runs
+    one wave a SIMD, with the covariate rows read by pairs (p = 1, 3) or one by
+    one (p = 5), and above 65,536 sites without pairs two waves.  B and F are
+    those of the form that evaluates C again, bit for bit."""
+    print(f"mixed m=16 cov={cov} n={n} p={p}", flush=True)
+    m = 16
+    c = uniform_coords(n, 7 + cov)
+    rng = np.random.default_rng(n + p)
+    X = np.column_stack([np.ones(n), rng.normal(size=(n, p - 1))])
+    beta = np.linspace(1.0, -1.0, p)
+    y = X @ beta + rng.normal(size=n)
+    nn = nngp.mkNNIndxCB(c, m)
+    theta = [2.0, 0.2, 12.0 if cov != 1 else 3.0] + ([1.5] if cov == 2 else [])
+    with nngp.Model(c, nn["nnIndx"], nn["nnIndxLU"], m, cov, X, y,
+                    precision=1) as md:
+        md.set_shape(0, 64, 0)
+        ref = md.update(theta, slot=0, beta=beta)
+        B0, F0 = md.get_bf(0)
+        for th in (64, 128, 256):
+            md.set_shape(0, th, 3)
+            out = md.update(theta, slot=0, beta=beta)
+            B, F = md.get_bf(0)
+            assert np.array_equal(B, B0) and np.array_equal(F, F0), th
+            for key in ("logDet", "qResid"):
+                assert abs(out[key] - ref[key]) < 1e-12 * abs(ref[key]), key
