@@ -484,7 +484,8 @@ int bf_rows(const BfArgs &a, const BfConfig &cfg) {
   // the row kernel's waves take groups of four sites
   const int units = cfg.family == 2 ? (a.n + 3) / 4 : a.n;
   const int need = (units + waves - 1) / waves;
-  const int most = cfg.family == 2 ? kGrpWaves / waves : kCoopBlocks;
+  const bool two = cfg.family == 2 && (a.m > 16 || a.c.cov == 2);
+  const int most = two ? kGrpWaves / waves : kCoopBlocks;
   return need < most ? need : most;
 }
 
