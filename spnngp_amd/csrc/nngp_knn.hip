@@ -750,17 +750,18 @@ int knn_build(const double *coords, int n, int m, int mode,
   return NNGP_OK;
 }
 
-// Queries up to which nn2 gives each a wavefront when k <= 16: about 4.5 us a
-// thousand queries, against 150 to 280 us for one query a lane whatever their
-// number (n = 2e3 to 1e6, k = 10 and 15).  For k > 16 the lanes' 32- and
+// Queries up to which nn2 gives each a wavefront when k <= 16.  That takes 17 us
+// and 3.1 us a thousand queries whatever k; one query a lane takes about 30 + 13
+// k us whatever their number (n = 2e3, 1e5 and 1e6: k = 1 42 to 64 us, k = 5 92
+// to 144, k = 10 141 to 192, k = 15 217 to 254).  For k > 16 the lanes' 32- and
 // 64-entry lists took 2 to 6 ms, against 7 us a thousand.
-constexpr int kNn2Wave = 49152;
+static int nn2_wave_queries(int k) { return std::min(4096 * (k + 1), 49152); }
 
 int nn2_launch(const Nn2Args &a, hipStream_t st) {
   if (a.nq <= 0) return 0;
   if (a.k > 64) return -1;
   const dim3 block(kKnnBlock);
-  if (a.k > 16 || a.nq <= kNn2Wave)
+  if (a.k > 16 || a.nq <= nn2_wave_queries(a.k))
     return wave_launches(a.nq, [&](int first, dim3 grid) {
       hipLaunchKernelGGL(k_nn2_wave, grid, block, 0, st, a, first);
     });

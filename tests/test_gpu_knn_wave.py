@@ -24,7 +24,8 @@ def test_predecessors_bit_exact(oracle, nngp, n, m, ordered):
 
 @pytest.mark.parametrize("n,k,q", [(1, 1, 3), (64, 64, 5), (65, 64, 70),
                                    (3000, 17, 400), (3000, 15, 49152),
-                                   (3000, 15, 49153)])
+                                   (3000, 15, 49153), (3000, 1, 8192),
+                                   (3000, 1, 8193), (3000, 5, 24577)])
 def test_nn2_bit_exact(oracle, nngp, n, k, q):
     print(f"nn2 wave n={n} k={k} q={q}", flush=True)
     rng = np.random.default_rng(n + k)
