@@ -8,7 +8,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("n,m", [(2, 1), (63, 62), (64, 15), (65, 63),
-                                 (129, 5), (1500, 63), (4097, 16)])
+                                 (129, 5), (1500, 63), (4097, 16),
+                                 (8192, 5), (8193, 5)])
 @pytest.mark.parametrize("ordered", [True, False])
 def test_predecessors_bit_exact(oracle, nngp, n, m, ordered):
     print(f"knn wave n={n} m={m} ordered={ordered}", flush=True)
@@ -33,6 +34,28 @@ def test_nn2_bit_exact(oracle, nngp, n, k, q):
     c0 = rng.uniform(-0.2, 1.2, size=(q, 2))  # some outside every strip
     i_ref, d_ref = oracle.nn2(c, c0, k)
     i_got, d_got = nngp.nn2(c, c0, k)
+    assert np.array_equal(i_got, i_ref) and np.array_equal(d_got, d_ref)
+
+
+@pytest.mark.parametrize("side", [7, 40, 95])
+def test_equal_coordinates_and_signed_zeros(oracle, nngp, side):
+    """Lattices in random order, on both sides of the number of points up to
+    which the strip index is counted instead of sorted: equal x and equal y, 0
+    and -0, and doubled sites."""
+    print(f"knn lattice {side} x {side}", flush=True)
+    g = np.arange(side) - side // 2
+    c = np.array([(x, y) for x in g for y in g], float) / 8.0
+    rng = np.random.default_rng(side)
+    c = np.vstack([c, c[rng.integers(0, len(c), 9)]])
+    c = rng.permutation(c)
+    c[(c == 0) & (rng.random(c.shape) < 0.5)] = -0.0
+    for got, want in ((nngp.mkNNIndxCB(c, 6), oracle.mkNNIndxCB(c, 6)),
+                      (nngp.mkNNIndx(c, 6), oracle.mkNNIndx(c, 6))):
+        for key in ("nnIndx", "nnIndxLU", "nnDist"):
+            assert np.array_equal(got[key], want[key]), key
+    q = rng.uniform(-side / 16, side / 16, size=(50, 2))
+    i_ref, d_ref = oracle.nn2(c, q, 9)
+    i_got, d_got = nngp.nn2(c, q, 9)
     assert np.array_equal(i_got, i_ref) and np.array_equal(d_got, d_ref)
 
 
