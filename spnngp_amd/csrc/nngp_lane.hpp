@@ -63,7 +63,9 @@ __host__ __device__ constexpr int lane_lds_entries(int M) {
 // B in the held-out sites and 36 B in the batched updateBF (none).  The single
 // updateBF pass at M = 15 has no spills without the mask and 12 B with it; at M
 // = 16 84 to 172 B without and 0 to 44 B with it (n = 3,000, p = 3, exponential:
-// 17.1 us, now 15.8; n = 1e6 241 and 210).
+// 17.1 us, now 15.8; n = 1e6 241 and 210).  Kriging at M = 8 takes 124 registers
+// without the mask and 136 with it, three waves a SIMD for four (2,000 sites x
+// 500 samples 59.9 and 63.0 us).
 template <int M, int K, bool HOOKS, bool EARLY, class Entry, class Rhs,
           class Mid, class Up>
 __device__ __forceinline__ bool lane_solve(double diag, Entry &&entry,

@@ -157,7 +157,7 @@ __global__ __launch_bounds__(kPredLane, 2) void k_pred_lane(PredArgs A) {
   const double nug = latent ? 0.0 : t2;
   double v[M];  // w
   double vv;
-  const bool ok = lane_solve<M, K, false, true>(
+  const bool ok = lane_solve<M, K, false, (M > 8)>(
       s2 * 1.0 + nug,
       [&](int k, int l) {
         return s2 *
