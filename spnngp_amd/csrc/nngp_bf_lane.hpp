@@ -78,7 +78,7 @@ __device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
   double2 z[ZH > 0 ? ZH : 1], zn[ZH > 0 ? M * ZH : 1];
   double v[M];  // B_i
   double vv;
-  const bool ok = lane_solve<M, K, (ZH > 0), (BATCH || M > 15)>(
+  const bool ok = lane_solve<M, K, (ZH > 0), ((BATCH && M > 8) || M > 15)>(
       c.diag,
       [&](int k, int l) {
         return lane_corr<COV>(lane_d2<COV>(px[k] - px[l], py[k] - py[l]), c);
@@ -129,10 +129,11 @@ __device__ __forceinline__ void lane_site(const BfArgs &A, const BfProblem &P,
       e[2 * h + 1] = z[h].y;
     }
   } else if (A.nz > 0) {
-    // the slots again (from cache), unless the registers held them at no cost
-    // in waves a SIMD: the second read is a round trip that a pass of few waves
-    // waits for (M = 8, n = 5e4: 11.7 us with it, 11.0 without)
-    if constexpr (BATCH || !(M <= 8 || M == 12)) {
+    // the slots again (from cache), unless the registers held them: the second
+    // read is a round trip that a pass of few waves waits for (M = 8, n = 5e4:
+    // 11.7 us with it, 11.0 without; batched, 150 problems of 4e4 sites, spherical:
+    // 338 and 302 us, at three waves a SIMD instead of four)
+    if constexpr (!(M <= 8 || (M == 12 && !BATCH))) {
 #pragma unroll
       for (int k = 0; k < M; k++) nb[k] = k < cnt ? P.nnIndx[off + k] : 0;
     }
