@@ -31,6 +31,7 @@ namespace nngp {
 
 constexpr int kSol = 96;        // per-problem solution record (doubles)
 constexpr int kSolA = 8, kSolB = 9, kSolOk = 10, kSolH = 16, kSolV = 32;
+constexpr int kCvPredThreads = 128;
 constexpr int kCvCoopWaves = 4;
 constexpr int kCvCoopBlocks = 512;
 
@@ -177,15 +178,9 @@ __device__ __forceinline__ double quad_vb(const double *Vb, const double *u,
   return q;
 }
 
-// Threads of a k_cv_pred_lane block for m neighbors: 128 where two waves a SIMD
-// need most of the registers or LDS, 256 for m <= 8 (150 problems of 1e4 sites,
-// m = 8: 126 us at 128, 120).
-__host__ __device__ constexpr int cv_threads(int m) { return m <= 8 ? 256 : 128; }
-
 // Waves of the largest block that sums its scores.
-constexpr int kCvMaxWaves = 4;
-static_assert(kCvMaxWaves >= kCvCoopWaves && 64 * kCvMaxWaves >= cv_threads(1),
-              "every wave has a place");
+constexpr int kCvMaxWaves =
+    kCvPredThreads / 64 > kCvCoopWaves ? kCvPredThreads / 64 : kCvCoopWaves;
 
 __device__ inline void block_pair_sum(double a, double b, double *prow,
                                       int cap, int row) {
@@ -213,22 +208,22 @@ __device__ inline void block_pair_sum(double a, double b, double *prow,
 // two-wave solve of the updateBF lane kernel (lane_solve): 250 problems of
 // 20,000 sites, m = 15, matern 3/2, took 1.67 ms with the triangle in
 // registers at one wave a SIMD; now 1.04 ms.  Up to M = 8 the registers hold the
-// neighbor slots through the solve (150 problems of 1e4 sites, M = 8: 142 us when
-// they were read again, now 120, 124 before lane_solve).
+// neighbor slots through the solve (150 problems, M = 8: 1e4 sites 142 us when
+// they were read again, now 126, and 1e3 sites 18 and 17; in 256-thread blocks
+// 120 and 28).
 template <int M, int COV>
-__global__ __launch_bounds__(cv_threads(M), 2) void k_cv_pred_lane(
+__global__ __launch_bounds__(kCvPredThreads, 2) void k_cv_pred_lane(
     CvPredArgs A) {
-  constexpr int kThreads = cv_threads(M);
   constexpr int K = lane_lds_entries(M);
-  __shared__ double2 area[K > 0 ? kThreads * K / 2 : 1];
-  const int nb = (A.nho + kThreads - 1) / kThreads;
+  __shared__ double2 area[K > 0 ? kCvPredThreads * K / 2 : 1];
+  const int nb = (A.nho + kCvPredThreads - 1) / kCvPredThreads;
   const int b = xcd_block(nb);
   if (b < 0) return;
   const int j = (int)blockIdx.y;
   const int f = __builtin_amdgcn_readfirstlane(j / A.ng);
   const CovArgs c = cov_uniform(A.covs + (j - f * A.ng));
   const double *so = A.sol + (size_t)j * kSol;
-  const int i = b * kThreads + (int)threadIdx.x;
+  const int i = b * kCvPredThreads + (int)threadIdx.x;
   double crps = 0.0, sq = 0.0;
   if (i < A.nho) {
     const double2 *xy = A.xy + (size_t)f * A.nmod;
@@ -406,8 +401,8 @@ __global__ __launch_bounds__(64 * kCvCoopWaves) void k_cv_pred_coop(
 }
 
 // Rows (logical blocks) per problem of the prediction launch.
-static int cv_pred_rows(int nho, int m, bool lane) {
-  if (lane) return (nho + cv_threads(m) - 1) / cv_threads(m);
+static int cv_pred_rows(int nho, bool lane) {
+  if (lane) return (nho + kCvPredThreads - 1) / kCvPredThreads;
   const int need = (nho + kCvCoopWaves - 1) / kCvCoopWaves;
   return need < kCvCoopBlocks ? need : kCvCoopBlocks;
 }
@@ -415,10 +410,10 @@ static int cv_pred_rows(int nho, int m, bool lane) {
 static int cv_pred_launch(CvPredArgs a, int variant, int nprob,
                           hipStream_t st) {
   const bool lane = a.m <= 16 && variant >= 0;
-  const int nrows = cv_pred_rows(a.nho, a.m, lane);
+  const int nrows = cv_pred_rows(a.nho, lane);
   const dim3 grid(8 * ((nrows + 7) / 8), nprob);
   if (lane) {
-    const dim3 blk(cv_threads(a.m));
+    const dim3 blk(kCvPredThreads);
 #define NNGP_CVP_COV(MM)                                                           \
   do {                                                                            \
     switch (variant) {                                                            \
@@ -668,7 +663,7 @@ int CvGrid::record(int g, int variant, bool want_y0) {
   if (!rc) rc = cv_pred_launch(pa, variant, nprob, st.s);
   if (!rc)
     rc = rows_sum_launch(prow.as<double>(), prow_cap,
-                         cv_pred_rows(nho, m, lane_pred), 2LL * prow_cap, 2,
+                         cv_pred_rows(nho, lane_pred), 2LL * prow_cap, 2,
                          nprob, pscore.as<double>(), 2, perr.as<int>(),
                          perrd.as<double>(), st.s);
   const hipError_t e = hipStreamEndCapture(st.s, &graph);
@@ -703,9 +698,9 @@ int CvGrid::run(const double *thetaAlpha, int g, double *scores,
   const int nv = 2 + nz * (nz + 1) / 2;
   if (nprob > cap_prob) {
     rows_cap = rows_capacity(nmod);
-    prow_cap = cv_pred_rows(nho, m, true) > cv_pred_rows(nho, m, false)
-                   ? cv_pred_rows(nho, m, true)
-                   : cv_pred_rows(nho, m, false);
+    prow_cap = cv_pred_rows(nho, true) > cv_pred_rows(nho, false)
+                   ? cv_pred_rows(nho, true)
+                   : cv_pred_rows(nho, false);
     NNGP_TRY(covs.alloc(sizeof(CovArgs) * (size_t)g));
     NNGP_TRY(rows.alloc(sizeof(double) * (size_t)nprob * nv * rows_cap));
     NNGP_TRY(sums.alloc(sizeof(double) * (size_t)nprob * kStatsMax));
