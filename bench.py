@@ -695,9 +695,8 @@ def chain_kernel(chosen, m, mixed=False, zs=4):
     M = 15 if m == 15 else m
     if mixed:
         if fam == "lane+reg-copy":
-            # rows staged (zs / 2 chunks) when the block's stage fits 64 KiB
-            stage = threads // 64 * (M + 1) * (zs // 2) * 64 * 16
-            zh = zs // 2 if m > 8 and stage <= 65536 else 0
+            # covariate rows by pairs, rows of two pairs up to 128 threads
+            zh = zs // 2 if m > 8 and (zs == 2 or threads <= 128) else 0
             return f"nngp::k_bf_mixed_reg<{M}, 0, {zh}> ({threads} threads)"
         if fam in ("lane", "lane+lds-copy"):
             copy = "true" if fam == "lane+lds-copy" else "false"

@@ -140,8 +140,8 @@ __host__ __device__ constexpr int site_terms(int nz) {
 // and combines its four partials (pairs, then the two pairs), and with more
 // than one wave per block the wave sums meet in LDS and are added in wave
 // order.  The order is fixed, so a launch shape's sums are reproducible.
-// `w` may be memory the wave has finished reading (the staged covariate
-// rows); the barrier before the writes also keeps those reads first.
+// `w` may be memory the wave has finished reading (the kept entries of its
+// factor); the barrier before the writes also keeps those reads first.
 __device__ inline void block_site_terms_lds(int nz, double *rows,
                                             int rows_cap, bool valid,
                                             double F,

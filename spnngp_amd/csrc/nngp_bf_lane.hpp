@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kLaneMaxThreads) void k_bf_lane(BfArgs A) {
 // m = 15, p = 3, exponential: 158 us a pass (20 iterations of a chain 3.71
 // ms) against 200 us (4.61 ms) with the triangle in registers at one wave and
 // the covariate rows staged in LDS; the vector units are busy 93% of the time
-// against 70%, at 4,257 instructions a wave against 4,660 (no moves to and
+// against 70%, at 4,286 instructions a wave against 4,660 (no moves to and
 // from the accumulation registers).  n = 4e5, mode 0 against 2: m = 9 57 and
 // 42 us, m = 12 74 and 54, m = 15 127 and 78, m = 16 145 and 97.
 template <int M, int COV, int ZH, bool BATCH>

@@ -452,10 +452,11 @@ static void launch_mixed_mc(const BfArgs &a, int variant, const dim3 &grid,
 }
 
 // Aligned pairs in a row of Z that k_bf_mixed_reg reads (zs = 2 ZH, Z 16-byte
-// aligned, m > 8), else 0: single values.
-static int mixed_reg_zh(const BfArgs &a) {
+// aligned, m > 8), else 0: single values, as also for rows of two pairs in
+// 256-thread blocks, a shape that smaller blocks beat.
+static int mixed_reg_zh(const BfArgs &a, int threads) {
   if (!a.Z || a.nz <= 0 || a.m <= 8 || ((uintptr_t)a.Z & 15) != 0) return 0;
-  return a.zs == 2 ? 1 : a.zs == 4 ? 2 : 0;
+  return a.zs == 2 ? 1 : a.zs == 4 && threads <= 128 ? 2 : 0;
 }
 
 // Sites up to which no SIMD of the 1,024 has a second wave.
@@ -465,6 +466,7 @@ template <int M, int ZH, int W>
 static void launch_mixed_reg_mhw(const BfArgs &a, int variant,
                                  const dim3 &grid, const dim3 &blk,
                                  hipStream_t st) {
+  // up to 72 KiB a block at 256 threads, which gfx950 grants (160 KiB a CU)
   const size_t shm = (size_t)(blk.x / 64) *
                      mixed_reg_wave_chunks(M, W, a.nz) * sizeof(double2);
   auto launch = [&](auto cov) {
@@ -506,7 +508,7 @@ static void launch_mixed_reg_mh(const BfArgs &a, int variant, const dim3 &grid,
 template <int M>
 static void launch_mixed_reg(const BfArgs &a, int variant, const dim3 &grid,
                              const dim3 &blk, hipStream_t st) {
-  switch (mixed_reg_zh(a)) {
+  switch (mixed_reg_zh(a, (int)blk.x)) {
     case 1: launch_mixed_reg_mh<M, 1>(a, variant, grid, blk, st); break;
     case 2: launch_mixed_reg_mh<M, 2>(a, variant, grid, blk, st); break;
     default: launch_mixed_reg_mh<M, 0>(a, variant, grid, blk, st); break;

@@ -463,9 +463,12 @@ __device__ __forceinline__ double matern_s2_fast(double d, const CovArgs &a,
 // the general-nu matern as a table in device memory (the row kernel)
 // ---------------------------------------------------------------------------
 // The same function on the same range [2^-30, 2^6) with each octave cut into
-// 16 equal pieces of the mantissa: the centre of a piece is at least 33
+// 16 equal pieces of the mantissa.  The centre of a piece is at least 33
 // half-widths from the singularity at 0, so the interpolant at 9 Chebyshev
-// points (degree 8) converges like 66^-9 = 4e-17.  Nine coefficients an
+// points (degree 8) is within 66^-9 = 4e-17 of it there; where the factor e^-x
+// decides (half-width h, error e^-x h^9 / (9! 2^8)), it is 3e-11 of the value at
+// x = 16 and 3e-8 at 32, but never more than 1.1e-17 of s2, which is what an
+// entry of C needs.  Nine coefficients an
 // entry instead of 16 matter because the row kernel is bound by its LDS
 // reads of them; the piece number is the exponent and the top four mantissa
 // bits of x, and a row of nine doubles puts neighboring pieces' k-th

@@ -106,9 +106,10 @@ def nn2(coords, coords0, k: int):
 def _shape_name(family, mode):
     """Name of an updateBF launch shape of the autotuner: 'lane' (one site
     per lane; '+lds-copy' and '+reg-copy' for the mixed form's covariance
-    copy in LDS or in registers, '+lds-z' for the FP64 form that keeps finished
-    rows of the factor in LDS), 'wave' (one site per wavefront) or 'row' (one site per
-    16-lane row, four per wavefront)."""
+    copy in LDS or in registers; '+lds-z', a name kept for callers that match
+    on it, for the FP64 form that keeps finished rows of the factor in LDS),
+    'wave' (one site per wavefront) or 'row' (one site per 16-lane row, four
+    per wavefront)."""
     if family == 0:
         return ("lane", "lane+lds-copy", "lane+lds-z", "lane+reg-copy")[mode]
     return "row" if family == 2 else "wave"

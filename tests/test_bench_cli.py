@@ -45,8 +45,8 @@ def test_chain_kernel_names_follow_the_launch_shapes():
     b = _bench()
     assert b.chain_kernel(("lane+lds-z", 64), 15) == \
         "nngp::k_bf_lane_lds<15, 0, 2, false> (64 threads)"
-    # the mixed register copy stages rows (zs = 4) while the block's stage
-    # fits 64 KiB: 64 and 128 threads, not 256
+    # the mixed register copy reads rows of two pairs (zs = 4) by pairs at 64
+    # and 128 threads, not 256
     assert b.chain_kernel(("lane+reg-copy", 128), 15, True, 4) == \
         "nngp::k_bf_mixed_reg<15, 0, 2> (128 threads)"
     assert b.chain_kernel(("lane+reg-copy", 256), 15, True, 4) == \

@@ -340,7 +340,7 @@ def test_set_shape_rejects_shapes_that_do_not_apply(nngp):
             md.set_shape(1, 96, 0)
         md.set_shape(1, 128, 0)
     # modes of the other precision: 1 and 3 are the mixed kernel's
-    # covariance copies, 2 the FP64 kernel's staged rows
+    # covariance copies, 2 the FP64 kernel's rows in LDS
     nn15 = nngp.mkNNIndxCB(c, 15)
     with nngp.Model(c, nn15["nnIndx"], nn15["nnIndxLU"], 15, 0) as md:
         for mode in (1, 3):
@@ -695,15 +695,14 @@ def test_mixed_updateBF_close_to_oracle(oracle, nngp, cov, m):
                                      (2, 10, 3), (2, 16, 2)])
 def test_mixed_lane_modes_agree(oracle, nngp, cov, m, p):
     """The mixed per-lane kernel's three ways to keep C for the refinement
-    residual (re-evaluated, LDS copy, register copy at one wave per SIMD
-    with the covariate rows staged in LDS where they can be) run the same
-    arithmetic: B and F equal bit for bit across modes and block sizes, and
-    the sums, added in another order by the register form, agree to
-    rounding.  n = 4000 + 13 leaves a ragged last block; p = 2 has rows
-    that stage in one 16-byte chunk, p = 1 and 0 none; at 256 threads the
-    register form's stage of p = 3 rows exceeds 64 KiB and it reads them
-    from memory.  The matern cases run the closed forms at nu = 1.5 and
-    2.5."""
+    residual (re-evaluated, LDS copy, register copy with a part of it in LDS
+    from m = 13 on) run the same arithmetic: B and F equal bit for bit across
+    modes and block sizes, and the sums, added in another order by the register
+    form, agree to rounding.  n = 4000 + 13 leaves a ragged last block; the
+    register form reads the covariate rows by aligned pairs (two at p = 2 and 3,
+    one at p = 1) for m > 8, rows of two pairs one value at a time at 256
+    threads, where its LDS takes 72 KiB a block.  The matern cases run the
+    closed forms at nu = 1.5 and 2.5."""
     print(f"mixed modes cov={cov} m={m} p={p}", flush=True)
     n = 4000 + 13
     c = uniform_coords(n, 60 + m + p)
