@@ -416,8 +416,9 @@ typedef struct nngp_tune_report {
   int mode[NNGP_TUNE_MAX];        /* family 0, NNGP_MIXED: 1 = the
                                      covariance copy kept in LDS for the
                                      refinement residual, 3 = kept in
-                                     registers and LDS (two waves per
-                                     SIMD), 0 = re-evaluated; family 0, FP64:
+                                     registers and LDS (two waves per SIMD;
+                                     at m = 16 one, in registers), 0 =
+                                     re-evaluated; family 0, FP64:
                                      2 = finished rows of the factor kept
                                      in LDS, two waves per SIMD (same
                                      results bit for bit as 0)            */

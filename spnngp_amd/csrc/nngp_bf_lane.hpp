@@ -199,7 +199,7 @@ __global__ __launch_bounds__(kLaneMaxThreads) void k_bf_lane(BfArgs A) {
 // the covariate rows staged in LDS; the vector units are busy 93% of the time
 // against 70%, at 4,286 instructions a wave against 4,660 (no moves to and
 // from the accumulation registers).  n = 4e5, mode 0 against 2: m = 9 57 and
-// 42 us, m = 12 74 and 54, m = 15 127 and 78, m = 16 145 and 97.
+// 42 us, m = 12 74 and 54, m = 15 127 and 78, m = 16 146 and 89.
 template <int M, int COV, int ZH, bool BATCH>
 __global__ __launch_bounds__(kLaneMaxThreads, 2) void k_bf_lane_lds(BfArgs A) {
   extern __shared__ double2 lane_lds[];
