@@ -697,7 +697,8 @@ def chain_kernel(chosen, m, mixed=False, zs=4):
         if fam == "lane+reg-copy":
             # covariate rows by pairs, rows of two pairs up to 128 threads
             zh = zs // 2 if m > 8 and (zs == 2 or threads <= 128) else 0
-            return f"nngp::k_bf_mixed_reg<{M}, 0, {zh}> ({threads} threads)"
+            form = "one" if m == 16 and zh else "reg"
+            return f"nngp::k_bf_mixed_{form}<{M}, 0, {zh}> ({threads} threads)"
         if fam in ("lane", "lane+lds-copy"):
             copy = "true" if fam == "lane+lds-copy" else "false"
             return f"nngp::k_bf_mixed<{M}, 0, {copy}> ({threads} threads)"
